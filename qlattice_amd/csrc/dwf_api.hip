@@ -1988,8 +1988,7 @@ void apply_full_dev(Inv& I, int op, double2* out_aos, const double2* in_aos)
   double2* io = W(I, W_IN_O);
   double2* oe = W(I, W_OUT_E);
   double2* oo = W(I, W_OUT_O);
-  qdwf::launch_pack5(in_aos, ie, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_pack5(in_aos, io, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_pack5_full(in_aos, ie, io, I.geo, I.ls, I.stream);
   check_launch();
   switch (op) {
     case F_M: op_m_full(I, oe, oo, ie, io); break;
@@ -1997,8 +1996,7 @@ void apply_full_dev(Inv& I, int op, double2* out_aos, const double2* in_aos)
     case F_DMINUS: op_d_minus(I, oe, oo, ie, io); break;
     default: throw ArgError("unknown operator");
   }
-  qdwf::launch_unpack5(oe, out_aos, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_unpack5(oo, out_aos, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_unpack5_full(oe, oo, out_aos, I.geo, I.ls, I.stream);
   check_launch();
 }
 
@@ -2022,12 +2020,10 @@ long invert_5d_dev(Inv& I, double2* out_aos, const double2* in_aos)
   double2* io = W(I, W_IN_O);
   double2* oe = W(I, W_OUT_E);
   double2* oo = W(I, W_OUT_O);
-  qdwf::launch_pack5(in_aos, ie, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_pack5(in_aos, io, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_pack5_full(in_aos, ie, io, I.geo, I.ls, I.stream);
   check_launch();
   const long it = invert_halves(I, ie, io, oe, oo);
-  qdwf::launch_unpack5(oe, out_aos, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_unpack5(oo, out_aos, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_unpack5_full(oe, oo, out_aos, I.geo, I.ls, I.stream);
   check_launch();
   return it;
 }
@@ -2259,13 +2255,11 @@ long invert_5d_batch_dev(qlat_dwf_inverter* const* invs, int n, double2* const* 
   return solve_columns(
       I, n, colinv.data(),
       [&](int j, Inv& J, double2* e, double2* o) {
-        qdwf::launch_pack5(src[j], e, J.geo, J.ls, 2, 1, J.stream);
-        qdwf::launch_pack5(src[j], o, J.geo, J.ls, 1, 1, J.stream);
+        qdwf::launch_pack5_full(src[j], e, o, J.geo, J.ls, J.stream);
         check_launch();
       },
       [&](int j, Inv& J, const double2* e, const double2* o) {
-        qdwf::launch_unpack5(e, sol[j], J.geo, J.ls, 2, 1, J.stream);
-        qdwf::launch_unpack5(o, sol[j], J.geo, J.ls, 1, 1, J.stream);
+        qdwf::launch_unpack5_full(e, o, sol[j], J.geo, J.ls, J.stream);
         check_launch();
       },
       iters);
@@ -2764,14 +2758,11 @@ long invert_5d_with_guess_dev(Inv& I, double2* out_aos, const double2* in_aos)
   double2* io = W(I, W_IN_O);
   double2* ge = W(I, W_G_E);
   double2* go = W(I, W_G_O);
-  qdwf::launch_pack5(in_aos, ie, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_pack5(in_aos, io, I.geo, I.ls, 1, 1, I.stream);
-  qdwf::launch_pack5(out_aos, ge, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_pack5(out_aos, go, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_pack5_full(in_aos, ie, io, I.geo, I.ls, I.stream);
+  qdwf::launch_pack5_full(out_aos, ge, go, I.geo, I.ls, I.stream);
   check_launch();
   const long it = invert_halves_with_guess(I, ie, io, ge, go);
-  qdwf::launch_unpack5(ge, out_aos, I.geo, I.ls, 2, 1, I.stream);
-  qdwf::launch_unpack5(go, out_aos, I.geo, I.ls, 1, 1, I.stream);
+  qdwf::launch_unpack5_full(ge, go, out_aos, I.geo, I.ls, I.stream);
   check_launch();
   return it;
 }

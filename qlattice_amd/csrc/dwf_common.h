@@ -252,6 +252,13 @@ __device__ __forceinline__ double2 load_nt(const double2* p)
   return make_double2(t.x, t.y);
 }
 
+template <bool NT>
+__device__ __forceinline__ double2 load_in(const double2* p)
+{
+  if constexpr (NT) return load_nt(p);
+  else return *p;
+}
+
 // ---------------------------------------------------------------- spinors
 template <class T>
 struct SpinorIO;

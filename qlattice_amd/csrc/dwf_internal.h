@@ -12,6 +12,15 @@ constexpr int kMaxBlasGrid = 2048;
 constexpr int kHopM5Sites = 32;  // output half-sites per fused hop + s-matrix block
 constexpr int kMaxRhs = 16;      // right-hand sides per multi-RHS launch (tile width)
 
+// Grid of a grid-stride kernel over n elements.
+inline int blas_grid(int64_t n)
+{
+  int64_t g = (n + kBlasBlock - 1) / kBlasBlock;
+  if (g > kMaxBlasGrid) g = kMaxBlasGrid;
+  if (g < 1) g = 1;
+  return (int)g;
+}
+
 // The columns a launch works on: column rhs[i] of a stack of fields spaced
 // fstride slots apart, i < n.  A single field is {1, fstride, {0}}.
 struct RhsSet {
@@ -342,6 +351,9 @@ void launch_f2d(const float4* in, double2* out, int ls, int64_t st, int acc, hip
 
 void launch_pack5(const double2* aos, double2* soa, const LatGeo& g, int ls, int eo, int full, hipStream_t st);
 void launch_unpack5(const double2* soa, double2* aos, const LatGeo& g, int ls, int eo, int full, hipStream_t st);
+void launch_pack5_full(const double2* aos, double2* even, double2* odd, const LatGeo& g, int ls, hipStream_t st);
+void launch_unpack5_full(const double2* even, const double2* odd, double2* aos, const LatGeo& g, int ls,
+                         hipStream_t st);
 void launch_prop_col_to_5d(const double2* src, double2* soa, const LatGeo& g, int ls, int eo, int col,
                            hipStream_t st);
 void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, int ls, int eo, int col,

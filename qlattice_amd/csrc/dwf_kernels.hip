@@ -1907,14 +1907,6 @@ __global__ void __launch_bounds__(kBlasBlock) k_copy(const S* __restrict__ x, S*
     y[i] = x[i];
 }
 
-static int blas_grid(int64_t n)
-{
-  int64_t g = (n + kBlasBlock - 1) / kBlasBlock;
-  if (g > kMaxBlasGrid) g = kMaxBlasGrid;
-  if (g < 1) g = 1;
-  return (int)g;
-}
-
 template <class S>
 void launch_norm2(const S* a, int64_t n, double* part, double* out, hipStream_t st)
 {
@@ -2012,142 +2004,6 @@ void launch_f2d(const float4* in, double2* out, int ls, int64_t st, int acc, hip
   const int64_t n = (int64_t)ls * 6 * st;
   hipLaunchKernelGGL(k_f2d, dim3(blas_grid(n)), dim3(kBlasBlock), 0, s, in, out, n, acc, scale);
 }
-
-// ============================================================ layouts
-// Reference 5D field AoS complex128 [site][s][12] (full, V sites) or
-// [half][s][12] (half field).  `full` selects which: for a full field the
-// half-site h of parity eo sits at full index of half_coord(h, eo).
-__global__ void __launch_bounds__(kBlasBlock) k_pack5(const double2* __restrict__ aos, double2* __restrict__ soa,
-                                                      LatGeo g, int ls, int eo, int full)
-{
-  const int64_t n = g.vh * ls * 12;
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    // i enumerates (s, k, h) with h fastest
-    const int64_t h = i % g.vh, q = i / g.vh;
-    const int64_t s = q / 12, k = q - s * 12;
-    // full field: reference site index; half field: reference half index
-    int x[4];
-    half_coord(g, h, eo, x);
-    const int64_t site = full ? full_index(g, x) : full_index(g, x) / 2;
-    soa[sidx<12>(ls, (int)s, (int)k, h)] = aos[(site * ls + s) * 12 + k];
-  }
-}
-
-__global__ void __launch_bounds__(kBlasBlock) k_unpack5(const double2* __restrict__ soa, double2* __restrict__ aos,
-                                                        LatGeo g, int ls, int eo, int full)
-{
-  const int64_t n = g.vh * ls * 12;
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    const int64_t h = i % g.vh, q = i / g.vh;
-    const int64_t s = q / 12, k = q - s * 12;
-    int x[4];
-    half_coord(g, h, eo, x);
-    const int64_t site = full ? full_index(g, x) : full_index(g, x) / 2;
-    aos[(site * ls + s) * 12 + k] = soa[sidx<12>(ls, (int)s, (int)k, h)];
-  }
-}
-
-void launch_pack5(const double2* aos, double2* soa, const LatGeo& g, int ls, int eo, int full, hipStream_t st)
-{
-  const int64_t n = g.vh * ls * 12;
-  hipLaunchKernelGGL(k_pack5, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, aos, soa, g, ls, eo, full);
-}
-void launch_unpack5(const double2* soa, double2* aos, const LatGeo& g, int ls, int eo, int full, hipStream_t st)
-{
-  const int64_t n = g.vh * ls * 12;
-  hipLaunchKernelGGL(k_unpack5, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, soa, aos, g, ls, eo, full);
-}
-
-// Propagator column j ([site][12 rows][12 cols] complex128) -> 5D half field
-// of parity eo: the chiral embedding of fermion_field_5d_from_4d
-// (qcd-prop.h:96-116) with upper = 0, lower = Ls-1 (qcd-prop.h:157):
-// spins 0,1 go to s = 0, spins 2,3 to s = Ls-1, everything else is zero.
-// With col < 0 the input is a 4D fermion field [site][12].
-__global__ void __launch_bounds__(kBlasBlock) k_prop_col_to_5d(const double2* __restrict__ src, double2* __restrict__ soa,
-                                                               LatGeo g, int ls, int eo, int col)
-{
-  const int64_t n = g.vh * ls * 12;
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    const int64_t h = i % g.vh, q = i / g.vh;
-    const int s = (int)(q / 12), k = (int)(q - (int64_t)(q / 12) * 12);
-    double2 v = make_double2(0.0, 0.0);
-    const bool take = (k < 6) ? (s == 0) : (s == ls - 1);
-    if (take) {
-      int x[4];
-      half_coord(g, h, eo, x);
-      const int64_t site = full_index(g, x);
-      v = (col >= 0) ? src[(site * 12 + k) * 12 + col] : src[site * 12 + k];
-    }
-    soa[sidx<12>(ls, s, k, h)] = v;
-  }
-}
-
-// 5D half field of parity eo -> propagator column j (fermion_field_4d_from_5d,
-// qcd-prop.h:118-138, upper = Ls-1, lower = 0, qcd-prop.h:164).
-__global__ void __launch_bounds__(kBlasBlock) k_5d_to_prop_col(const double2* __restrict__ soa, double2* __restrict__ dst,
-                                                               LatGeo g, int ls, int eo, int col)
-{
-  const int64_t n = g.vh * 12;
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    const int64_t h = i % g.vh;
-    const int k = (int)(i / g.vh);
-    const int s = (k < 6) ? ls - 1 : 0;
-    int x[4];
-    half_coord(g, h, eo, x);
-    const int64_t site = full_index(g, x);
-    const double2 v = soa[sidx<12>(ls, s, k, h)];
-    if (col >= 0) dst[(site * 12 + k) * 12 + col] = v;
-    else dst[site * 12 + k] = v;
-  }
-}
-
-void launch_prop_col_to_5d(const double2* src, double2* soa, const LatGeo& g, int ls, int eo, int col, hipStream_t st)
-{
-  const int64_t n = g.vh * ls * 12;
-  hipLaunchKernelGGL(k_prop_col_to_5d, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, src, soa, g, ls, eo, col);
-}
-void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, int ls, int eo, int col, hipStream_t st)
-{
-  const int64_t n = g.vh * 12;
-  hipLaunchKernelGGL(k_5d_to_prop_col, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, soa, dst, g, ls, eo, col);
-}
-
-// Gauge AoS [site][mu][3][3] complex128 -> per-output-parity 8-link layout
-// (dwf_common.h), FP64 and FP32 copies.  Backward links are stored already
-// adjointed: U_mu(x - mu)^+.
-__global__ void __launch_bounds__(kBlasBlock) k_pack_gauge(const double2* __restrict__ gauge, double2* __restrict__ l64,
-                                                           float2* __restrict__ l32, unsigned* __restrict__ l16,
-                                                           LatGeo g)
-{
-  const int64_t n = g.vh * 2 * 8;
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    const int64_t h = i % g.vh, q = i / g.vh;
-    const int p = (int)(q / 8), d = (int)(q % 8);
-    const int eo = (p == 0) ? 2 : 1;
-    int x[4];
-    half_coord(g, h, eo, x);
-    const int mu = d & 3;
-    if (d >= 4) x[mu] = wrap_dec(x[mu], g.n[mu]);
-    const int64_t site = full_index(g, x);
-    const double2* U = &gauge[(site * 4 + mu) * 9];
-    for (int r = 0; r < 3; ++r)
-      for (int c = 0; c < 3; ++c) {
-        double2 v = (d < 4) ? U[r * 3 + c] : make_double2(U[c * 3 + r].x, -U[c * 3 + r].y);
-        const int64_t off = lidx(g.stride, p, d * 9 + r * 3 + c, h);
-        l64[off] = v;
-        l32[off] = make_float2((float)v.x, (float)v.y);
-        if (l16) l16[off] = pack_h2((float)v.x, (float)v.y);
-      }
-  }
-}
-
-void launch_pack_gauge(const double2* gauge, double2* l64, float2* l32, unsigned* l16, const LatGeo& g,
-                       hipStream_t st)
-{
-  const int64_t n = g.vh * 16;
-  hipLaunchKernelGGL(k_pack_gauge, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, gauge, l64, l32, l16, g);
-}
-
 
 // ------------------------------------------------------------ RngState fill
 // SHA-256 (FIPS 180-4): the round constants and one compression of a
