@@ -183,10 +183,9 @@ struct qlat_dwf_inverter {
   long max_cycle = 300;
   int solver = QLAT_DWF_SOLVER_FP64;
   double delta = 0.01;
-  // hop launch shapes (launch_hop): LDS-staged links; FP64 with streaming stores
-  int hop_spt64 = -102, hop_spt32 = -4;
+  // FP32 hop launch shape (launch_hop): LDS-staged links
+  int hop_spt32 = -4;
   bool fused32 = true;  // FP32 hop + s-matrix fusion (QLAT_DWF_FUSED=0 disables)
-  bool fused64 = true;  // FP64 hop + s-matrix fusion, k_hop_m5d (QLAT_DWF_FUSED64=0 disables)
   bool three_phase32 = true;   // FP32 solver on the three-phase kernels (QLAT_DWF_THREE_PHASE=0: fused
                                // FP32 kernels, single s-matrix pass per hop)
   int tp_sb = 32;              // sites per block of the three-phase kernels (QLAT_DWF_TP_SB)
@@ -228,6 +227,12 @@ struct qlat_dwf_inverter {
   // Off by default: measured at most 2.5% faster (8^3x16) and 1-5% slower
   // from 12^3x24 up, where a host round trip is a small part of an iteration.
   int graph_iters = 0;
+  // FP64 CG: scalars of two iterations, their mapped host copy, the events
+  // of the two groups of iterations in flight
+  qdwf::CgState64* cg64 = nullptr;
+  qdwf::CgState64* cg64_map = nullptr;
+  qdwf::CgState64* cg64_map_dev = nullptr;
+  hipEvent_t cg64_ev[2] = {nullptr, nullptr};
   qdwf::CgState* cg_dev = nullptr;
   qdwf::CgState* cg_host = nullptr;
 
@@ -407,7 +412,6 @@ struct Prec<double> {
   static const cplx<double>* mat(const Inv& I, int id) { return I.mat64 + (size_t)id * 2 * I.ls * I.ls; }
   static const cplx<double>* beta(const Inv& I, int which) { return I.beta64 + (size_t)which * I.ls; }
   static const void* links(const Inv& I) { return I.l64; }
-  static int spt(const Inv& I) { return I.hop_spt64; }
   static int64_t n(const Inv& I) { return n64(I); }
 };
 template <>
@@ -416,7 +420,6 @@ struct Prec<float> {
   static const cplx<float>* mat(const Inv& I, int id) { return I.mat32 + (size_t)id * 2 * I.ls * I.ls; }
   static const cplx<float>* beta(const Inv& I, int which) { return I.beta32 + (size_t)which * I.ls; }
   static const void* links(const Inv& I) { return I.l32; }
-  static int spt(const Inv& I) { return I.hop_spt32; }
   static int64_t n(const Inv& I) { return n32(I); }
 };
 
@@ -449,16 +452,19 @@ void m5(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, i
   a.in = in;
   a.out = out;
   a.x = x;
-  qdwf::launch_m5<T>(a, I.stream);
+  if constexpr (std::is_same<T, double>::value) qdwf::launch_smat_d(a, I.stream);
+  else qdwf::launch_m5<T>(a, I.stream);
   check_launch();
 }
 
 // out(parity eo_out) = alpha * H in + beta_s * x   (beta: 0 ones, 1 c~)
 template <class T>
 void hop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, int eo_out, bool dag,
-         T alpha = 1, const typename Prec<T>::slot* x = nullptr, int beta = 0, const qdwf::RhsSet* cols = nullptr)
+         T alpha = 1, const typename Prec<T>::slot* x = nullptr, int beta = 0, const qdwf::RhsSet* cols = nullptr,
+         const qdwf::CgState64* cg = nullptr)
 {
   qdwf::HopArgs<T> a;
+  a.cg = cg;
   a.cols = cols ? *cols : one_col();
   a.geo = I.geo;
   a.ls = I.ls;
@@ -470,7 +476,8 @@ void hop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, 
   a.x = x;
   a.beta = Prec<T>::beta(I, beta);
   a.links = Prec<T>::links(I);
-  qdwf::launch_hop<T>(a, dag, Prec<T>::spt(I), I.stream);
+  if constexpr (std::is_same<T, double>::value) qdwf::launch_hop_d(a, dag, I.stream);
+  else qdwf::launch_hop<T>(a, dag, I.hop_spt32, I.stream);
   check_launch();
 }
 
@@ -537,11 +544,11 @@ bool hop_m5_32(Inv& I, float4* out, const float4* in, int eo_out, bool dag, int 
   return true;
 }
 
-// FP64 fused out = alpha * Mat (H in) + beta * x (false if not available)
-bool hop_m5_64(Inv& I, double2* out, const double2* in, int eo_out, bool dag, int mat, double alpha = 1.0,
-               const double2* x = nullptr, double beta = 0.0, const double2* dotp = nullptr)
+// FP64 fused out = alpha * Mat (H in) + beta * x
+void hop_m5_64(Inv& I, double2* out, const double2* in, int eo_out, bool dag, int mat, double alpha = 1.0,
+               const double2* x = nullptr, double beta = 0.0, const double2* dotp = nullptr,
+               const qdwf::CgState64* cg = nullptr)
 {
-  if (!I.fused64) return false;
   qdwf::HopM5dArgs a{};
   a.geo = I.geo;
   a.ls = I.ls;
@@ -556,9 +563,9 @@ bool hop_m5_64(Inv& I, double2* out, const double2* in, int eo_out, bool dag, in
   a.real_mat = I.real_mat[mat];
   a.dotp = dotp;
   a.part = I.part;
-  if (!qdwf::launch_hop_m5d(a, dag, I.stream)) return false;
+  a.cg = cg;
+  if (!qdwf::launch_hop_m5d(a, dag, I.stream)) throw std::logic_error("internal: no FP64 hop kernel of this form");
   check_launch();
-  return true;
 }
 
 // Mpc = 1 - H K H K
@@ -574,10 +581,9 @@ void op_mpc(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* i
       return;
     }
   } else {
-    if (hop_m5_64(I, t2, t1, 3 - eo, false, MAT_K)) {
-      hop<T>(I, out, t2, eo, false, (T)-1, in, 0);
-      return;
-    }
+    hop_m5_64(I, t2, t1, 3 - eo, false, MAT_K);
+    hop<T>(I, out, t2, eo, false, (T)-1, in, 0);
+    return;
   }
   hop<T>(I, t2, t1, 3 - eo, false);
   m5<T>(I, t1, t2, MAT_K);
@@ -596,10 +602,9 @@ void op_mpcdag(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot
       return;
     }
   } else {
-    if (hop_m5_64(I, t2, in, 3 - eo, true, MAT_K_DAG)) {
-      hop_m5_64(I, out, t2, eo, true, MAT_K_DAG, -1.0, in, 1.0);
-      return;
-    }
+    hop_m5_64(I, t2, in, 3 - eo, true, MAT_K_DAG);
+    hop_m5_64(I, out, t2, eo, true, MAT_K_DAG, -1.0, in, 1.0);
+    return;
   }
   hop<T>(I, t1, in, 3 - eo, true);
   m5<T>(I, t2, t1, MAT_K_DAG);
@@ -616,43 +621,27 @@ void op_hermop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot
   op_mpcdag<T>(I, out, y, eo);
 }
 
-// CG form of Mpc^+ Mpc: ap = A p given t1 = K p (computed by the previous
-// CG step), with Re <p, ap> reduced in the same pass, for every column of
-// `cols` (stacks of fields).  dots[i] receives column i's value.
-template <class T>
-void hermop_t1_dot(Inv& I, typename Prec<T>::slot* ap, const typename Prec<T>::slot* p,
-                   const typename Prec<T>::slot* t1, int eo, const qdwf::RhsSet& cols,
-                   typename Prec<T>::slot* A, typename Prec<T>::slot* B, typename Prec<T>::slot* Y, double* dots)
+// CG form of Mpc^+ Mpc in FP32: ap = A p given t1 = K p (computed by the
+// previous CG step), with Re <p, ap> reduced in the same pass, for every
+// column of `cols` (stacks of fields).  dots[i] receives column i's value.
+void hermop_t1_dot(Inv& I, float4* ap, const float4* p, const float4* t1, int eo, const qdwf::RhsSet& cols, float4* A,
+                   float4* B, float4* Y, double* dots)
 {
   int64_t nparts = 0;
-  bool done = false;
-  if constexpr (std::is_same<T, float>::value) {
-    if (hop_m5_32(I, B, t1, 3 - eo, false, MAT_K, 1.f, nullptr, 0.f, nullptr, &cols)) {
-      hop<T>(I, Y, B, eo, false, (T)-1, p, 0, &cols);                         // y = p - H K H K p
-      hop_m5_32(I, B, Y, 3 - eo, true, MAT_K_DAG, 1.f, nullptr, 0.f, nullptr, &cols);  // u = K^+ H^+ y
-      hop_m5_32(I, ap, B, eo, true, MAT_K_DAG, -1.f, Y, 1.f, p, &cols);      // ap = y - K^+ H^+ u
-      nparts = qdwf::hop_m5_blocks(I.geo);
-      done = true;
-    }
+  if (hop_m5_32(I, B, t1, 3 - eo, false, MAT_K, 1.f, nullptr, 0.f, nullptr, &cols)) {
+    hop<float>(I, Y, B, eo, false, -1.f, p, 0, &cols);                               // y = p - H K H K p
+    hop_m5_32(I, B, Y, 3 - eo, true, MAT_K_DAG, 1.f, nullptr, 0.f, nullptr, &cols);  // u = K^+ H^+ y
+    hop_m5_32(I, ap, B, eo, true, MAT_K_DAG, -1.f, Y, 1.f, p, &cols);                // ap = y - K^+ H^+ u
+    nparts = qdwf::hop_m5_blocks(I.geo);
   } else {
-    if (cols.n == 1 && cols.rhs[0] == 0 && I.fused64 && qdwf::hop_m5d_ok(I.ls)) {
-      hop_m5_64(I, B, t1, 3 - eo, false, MAT_K);                      // b = K H K p
-      hop<T>(I, Y, B, eo, false, (T)-1, p, 0, &cols);                  // y = p - H b
-      hop_m5_64(I, B, Y, 3 - eo, true, MAT_K_DAG);                     // u = K^+ H^+ y
-      hop_m5_64(I, ap, B, eo, true, MAT_K_DAG, -1.0, Y, 1.0, p);       // ap = y - K^+ H^+ u
-      nparts = qdwf::hop_m5d_blocks(I.geo);
-      done = true;
-    }
-  }
-  if (!done) {
-    hop<T>(I, A, t1, 3 - eo, false, (T)1, nullptr, 0, &cols);
-    m5<T>(I, B, A, MAT_K, (T)1, nullptr, (T)0, nullptr, &cols);
-    hop<T>(I, Y, B, eo, false, (T)-1, p, 0, &cols);
-    hop<T>(I, A, Y, 3 - eo, true, (T)1, nullptr, 0, &cols);
-    m5<T>(I, B, A, MAT_K_DAG, (T)1, nullptr, (T)0, nullptr, &cols);
-    hop<T>(I, A, B, eo, true, (T)1, nullptr, 0, &cols);
-    m5<T>(I, ap, A, MAT_K_DAG, (T)-1, Y, (T)1, p, &cols);
-    nparts = (I.geo.vh + qdwf::kM5Block - 1) / qdwf::kM5Block * qdwf::SpinorIO<T>::kSlots;
+    hop<float>(I, A, t1, 3 - eo, false, 1.f, nullptr, 0, &cols);
+    m5<float>(I, B, A, MAT_K, 1.f, nullptr, 0.f, nullptr, &cols);
+    hop<float>(I, Y, B, eo, false, -1.f, p, 0, &cols);
+    hop<float>(I, A, Y, 3 - eo, true, 1.f, nullptr, 0, &cols);
+    m5<float>(I, B, A, MAT_K_DAG, 1.f, nullptr, 0.f, nullptr, &cols);
+    hop<float>(I, A, B, eo, true, 1.f, nullptr, 0, &cols);
+    m5<float>(I, ap, A, MAT_K_DAG, -1.f, Y, 1.f, p, &cols);
+    nparts = (I.geo.vh + qdwf::kM5Block - 1) / qdwf::kM5Block * qdwf::SpinorIO<float>::kSlots;
   }
   qdwf::launch_reduce_rows(I.part, (int)nparts, cols.n, I.red_map_dev, I.stream);
   check_launch();
@@ -661,22 +650,32 @@ void hermop_t1_dot(Inv& I, typename Prec<T>::slot* ap, const typename Prec<T>::s
 }
 
 // single-field form
-template <class T>
-double hermop_t1_dot(Inv& I, typename Prec<T>::slot* ap, const typename Prec<T>::slot* p,
-                     const typename Prec<T>::slot* t1, int eo)
+double hermop_t1_dot(Inv& I, float4* ap, const float4* p, const float4* t1, int eo)
 {
   double d = 0;
   const qdwf::RhsSet c = one_col();
-  hermop_t1_dot<T>(I, ap, p, t1, eo, c, Tmp<T>::t2(I), Tmp<T>::t3(I), Tmp<T>::y(I), &d);
+  hermop_t1_dot(I, ap, p, t1, eo, c, Tmp<float>::t2(I), Tmp<float>::t3(I), Tmp<float>::y(I), &d);
   return d;
 }
 
-// x_i += alpha_i p_i (x may be null); p_i = r_i + beta_i p_i; t_i = K p_i
-template <class T>
-void cg_step(Inv& I, typename Prec<T>::slot* x, typename Prec<T>::slot* p, const typename Prec<T>::slot* r,
-             typename Prec<T>::slot* t, const double* alpha, const double* beta, const qdwf::RhsSet& cols)
+// The FP64 CG form: ap = A p given t1 = K p, with the block sums of
+// Re <p, ap> in I.part (hop_m5d_blocks of them); nothing is done once *cg
+// says so.
+void hermop_t1_dot64(Inv& I, double2* ap, const double2* p, const double2* t1, int eo, const qdwf::CgState64* cg)
 {
-  qdwf::CgStepArgs<T> a{};
+  double2* B = W(I, W_OP_T3);
+  double2* Y = W(I, W_OP_Y);
+  hop_m5_64(I, B, t1, 3 - eo, false, MAT_K, 1.0, nullptr, 0.0, nullptr, cg);  // b = K H K p
+  hop<double>(I, Y, B, eo, false, -1.0, p, 0, nullptr, cg);                    // y = p - H b
+  hop_m5_64(I, B, Y, 3 - eo, true, MAT_K_DAG, 1.0, nullptr, 0.0, nullptr, cg); // u = K^+ H^+ y
+  hop_m5_64(I, ap, B, eo, true, MAT_K_DAG, -1.0, Y, 1.0, p, cg);               // ap = y - K^+ H^+ u
+}
+
+// x_i += alpha_i p_i (x may be null); p_i = r_i + beta_i p_i; t_i = K p_i
+void cg_step(Inv& I, float4* x, float4* p, const float4* r, float4* t, const double* alpha, const double* beta,
+             const qdwf::RhsSet& cols)
+{
+  qdwf::CgStepArgs<float> a{};
   a.geo = I.geo;
   a.ls = I.ls;
   for (int i = 0; i < qdwf::kMaxRhs; ++i) {
@@ -684,21 +683,19 @@ void cg_step(Inv& I, typename Prec<T>::slot* x, typename Prec<T>::slot* p, const
     a.beta[i] = i < cols.n ? beta[i] : 0.0;
   }
   a.cols = cols;
-  a.mat = Prec<T>::mat(I, MAT_K);
+  a.mat = Prec<float>::mat(I, MAT_K);
   a.real_mat = I.real_mat[MAT_K];
   a.x = x;
   a.p = p;
-  a.r = const_cast<typename Prec<T>::slot*>(r);  // read only in this form
+  a.r = const_cast<float4*>(r);  // read only in this form
   a.t = t;
-  qdwf::launch_cg_step<T>(a, I.stream);
+  qdwf::launch_cg_step<float>(a, I.stream);
   check_launch();
 }
 
-template <class T>
-void cg_step(Inv& I, typename Prec<T>::slot* x, typename Prec<T>::slot* p, const typename Prec<T>::slot* r,
-             typename Prec<T>::slot* t, double alpha, double beta)
+void cg_step(Inv& I, float4* x, float4* p, const float4* r, float4* t, double alpha, double beta)
 {
-  cg_step<T>(I, x, p, r, t, &alpha, &beta, one_col());
+  cg_step(I, x, p, r, t, &alpha, &beta, one_col());
 }
 
 // ------------------------------------------------------------ BLAS-1
@@ -794,26 +791,65 @@ long cg_fp64(Inv& I, double2* x, const double2* b, double stop_rsd, long max_num
   copy64(I, p, r);
   m5<double>(I, t, p, MAT_K);
   const double qnorm_in = dev_norm2(I, b);
-  double qnorm_r = dev_norm2(I, r);
-  for (long iter = 1; iter <= max_num_iter; ++iter) {
-    // alpha = |r|^2 / Re <p, A p> ; r -= alpha A p (dslash.h:365-374)
-    const double pap = hermop_t1_dot<double>(I, ap, p, t, 1);
-    I.stats.hermop_fp64 += 1;
-    const double alpha = qnorm_r / pap;
-    qdwf::launch_axpy_norm<double2>(alpha, ap, r, n, I.part, I.red_map_dev, I.stream);
-    check_launch();
-    sync(I);
-    const double new_qnorm_r = I.red_map[0];
-    if (!std::isfinite(new_qnorm_r)) throw std::runtime_error("CG breakdown: non-finite residual (FP64)");
-    if (new_qnorm_r <= qnorm_in * stop_rsd * stop_rsd) {
-      qdwf::launch_axpy<double2>(alpha, p, x, n, I.stream);
+  const double qnorm_r = dev_norm2(I, r);
+  // The iteration's scalars stay on the device (dslash.h:365-392: alpha =
+  // |r|^2 / Re <p, A p>, r -= alpha A p, x += alpha p, beta, p = r + beta p),
+  // and iterations are queued kCgAhead at a time, one group ahead of the one
+  // the host waits for; those behind the converged one find its state and do
+  // nothing.  8^3x16 Ls8, whose iteration is 65 us of kernels: the solve
+  // 18.0 -> 10.7 ms.
+  constexpr int kCgAhead = 2;
+  if (!I.cg64) {
+    I.cg64 = (qdwf::CgState64*)dev_alloc(2 * sizeof(qdwf::CgState64));
+    QDWF_HIP(hipHostMalloc((void**)&I.cg64_map, sizeof(qdwf::CgState64), hipHostMallocMapped | hipHostMallocCoherent));
+    QDWF_HIP(hipHostGetDevicePointer((void**)&I.cg64_map_dev, I.cg64_map, 0));
+    for (auto& e : I.cg64_ev) QDWF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  *I.cg64_map = qdwf::CgState64{};
+  qdwf::launch_cg_init_d(I.cg64, qnorm_r, qnorm_in * stop_rsd * stop_rsd, I.stream);
+  check_launch();
+  // sums of many blocks go through a reduction kernel first
+  const int64_t nblk = qdwf::hop_m5d_blocks(I.geo, I.ls);
+  const bool reduce = nblk > 4096;
+  qdwf::CgIterDArgs ia{};
+  ia.geo = I.geo;
+  ia.ls = I.ls;
+  ia.mat = Prec<double>::mat(I, MAT_K);
+  ia.real_mat = I.real_mat[MAT_K];
+  ia.x = x;
+  ia.p = p;
+  ia.r = r;
+  ia.t = t;
+  ia.ap = ap;
+  ia.pap = reduce ? I.red : I.part;
+  ia.npap = reduce ? 1 : (int)nblk;
+  ia.rnorm = I.part + nblk;
+  ia.st = I.cg64;
+  ia.host = I.cg64_map_dev;
+  long queued = 0;
+  auto queue_group = [&](hipEvent_t ev) {
+    for (int j = 0; j < kCgAhead && queued < max_num_iter; ++j, ++queued) {
+      ia.slot = (int)(queued & 1);
+      hermop_t1_dot64(I, ap, p, t, 1, I.cg64 + ia.slot);
+      if (reduce) qdwf::launch_reduce_rows(I.part, (int)nblk, 1, I.red, I.stream);
+      qdwf::launch_cg_iter_d(ia, I.stream);
       check_launch();
-      return iter;
     }
-    // x += alpha p ; p = r + beta p ; t = K p (dslash.h:369-392)
-    const double beta = new_qnorm_r / qnorm_r;
-    cg_step<double>(I, x, p, r, t, alpha, beta);
-    qnorm_r = new_qnorm_r;
+    QDWF_HIP(hipEventRecord(ev, I.stream));
+  };
+  queue_group(I.cg64_ev[0]);
+  for (long g = 1;; ++g) {
+    const bool last = queued >= max_num_iter;
+    if (!last) queue_group(I.cg64_ev[g & 1]);
+    QDWF_HIP(hipEventSynchronize(I.cg64_ev[(g - 1) & 1]));
+    if (*(volatile int*)&I.cg64_map->done || last) {
+      sync(I);  // the groups queued behind
+      const qdwf::CgState64 end = *I.cg64_map;
+      I.stats.hermop_fp64 += end.iter;
+      if (end.done == 2) throw std::runtime_error("CG breakdown: non-finite residual (FP64)");
+      if (end.done) return (long)end.iter;
+      break;
+    }
   }
   return max_num_iter + 1;
 }
@@ -858,7 +894,7 @@ long cg_mixed(Inv& I, double2* x64, const double2* b64, double stop_rsd, long ma
   const double d2 = I.delta * I.delta;
   long iter = 0;
   while (iter < max_total_iter) {
-    const double pap = hermop_t1_dot<float>(I, ap, p, t, 1);
+    const double pap = hermop_t1_dot(I, ap, p, t, 1);
     I.stats.hermop_low += 1;
     const double alpha = rr / pap;
     qdwf::launch_axpy_norm<float4>(alpha, ap, r, n, I.part, I.red_map_dev, I.stream);
@@ -883,9 +919,9 @@ long cg_mixed(Inv& I, double2* x64, const double2* b64, double stop_rsd, long ma
       check_launch();
       rr_new = rr_true;
       maxrr = rr_true;
-      cg_step<float>(I, nullptr, p, r, t, 0.0, rr_new / rr);
+      cg_step(I, nullptr, p, r, t, 0.0, rr_new / rr);
     } else {
-      cg_step<float>(I, x, p, r, t, alpha, rr_new / rr);
+      cg_step(I, x, p, r, t, alpha, rr_new / rr);
     }
     rr = rr_new;
   }
@@ -969,7 +1005,7 @@ long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
   long it = 0;
   while (!active.empty() && it < cap) {
     const qdwf::RhsSet cs = colset(active);
-    hermop_t1_dot<float>(I, AP, P, T, 1, cs, A, B, Y, pap);
+    hermop_t1_dot(I, AP, P, T, 1, cs, A, B, Y, pap);
     I.stats.hermop_low += cs.n;
     qdwf::AxpyNormArgs<float4> an;
     an.ap = AP;
@@ -1019,7 +1055,7 @@ long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
     }
     if (!keep.empty()) {
       const qdwf::RhsSet ks = colset(keep);
-      cg_step<float>(I, X, P, R, T, ka.data(), kb.data(), ks);
+      cg_step(I, X, P, R, T, ka.data(), kb.data(), ks);
     }
     active.swap(keep);
   }
@@ -2418,6 +2454,10 @@ void free_all(Inv* I)
   f(I->part);
   f(I->red);
   if (I->red_map) (void)hipHostFree(I->red_map);
+  f(I->cg64);
+  if (I->cg64_map) (void)hipHostFree(I->cg64_map);
+  for (auto e : I->cg64_ev)
+    if (e) (void)hipEventDestroy(e);
   f(I->cg_dev);
   if (I->cg_host) (void)hipHostFree(I->cg_host);
   f(I->lm_basis);
@@ -2524,11 +2564,9 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
     QDWF_HIP(hipStreamSynchronize(I->stream));
     QDWF_HIP(hipFree(g));
     build_matrices(*I);
-    // hop launch shape: QLAT_DWF_HOP_SPT32 / QLAT_DWF_HOP_SPT64 (see launch_hop)
+    // FP32 hop launch shape: QLAT_DWF_HOP_SPT32 (see launch_hop)
     if (const char* e = std::getenv("QLAT_DWF_HOP_SPT32")) I->hop_spt32 = std::atoi(e);
-    if (const char* e = std::getenv("QLAT_DWF_HOP_SPT64")) I->hop_spt64 = std::atoi(e);
     if (const char* e = std::getenv("QLAT_DWF_FUSED")) I->fused32 = std::atoi(e) != 0;
-    if (const char* e = std::getenv("QLAT_DWF_FUSED64")) I->fused64 = std::atoi(e) != 0;
     if (const char* e = std::getenv("QLAT_DWF_THREE_PHASE")) I->three_phase32 = std::atoi(e) != 0;
     if (const char* e = std::getenv("QLAT_DWF_RHS_TILE")) I->rhs_tile = std::max(0, std::min(qdwf::kMaxRhs, std::atoi(e)));
     if (const char* e = std::getenv("QLAT_DWF_TP_SB")) {

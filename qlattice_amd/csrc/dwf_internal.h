@@ -42,6 +42,7 @@ struct HopArgs {
   const cplx<T>* beta; // per-s xpay coefficients (device), used with x
   const void* links;   // 8-link layout (dwf_common.h)
   RhsSet cols;         // in/out/x are stacks of fields
+  const void* cg;      // FP64: optional CgState64, nothing is done once it is done
 };
 
 template <class T>
@@ -155,8 +156,19 @@ struct HopM5Args {
   const CgState* cg;  // optional: blocks of columns with cg->mode != 0 do nothing
 };
 
+// Scalars of the FP64 CG on the device, one slot for the even and one for
+// the odd iterations: an iteration reads slot it & 1 and writes the other.
+struct CgState64 {
+  double rr;      // |r|^2 before the iteration
+  double target;  // stop when |r|^2 <= target
+  double alpha;   // of the iteration (k_cg_residual_d)
+  int64_t iter;   // iterations done before this one
+  int done;       // 0 running, 1 converged, 2 non-finite
+};
+
 // FP64 fused hop + s-matrix (k_hop_m5d): out = alpha * Mat (H in) + beta * x
-// on one FP64 field; with dotp (dagger xpay form) part[block] = Re <dotp, out>.
+// on one FP64 field; with dotp (dagger xpay form) part[block] = Re <dotp,
+// out>, hop_m5d_blocks of them.
 struct HopM5dArgs {
   LatGeo geo;
   int ls;
@@ -170,12 +182,33 @@ struct HopM5dArgs {
   bool real_mat;
   const double2* dotp;  // optional
   double* part;
+  const CgState64* cg;  // optional: nothing is done once cg->done
 };
-// false (nothing launched) when ls does not fit (4 <= ls <= 16, 16 ls a
-// multiple of 64) or the form is not available
+// any ls <= 32; false (nothing launched) for a form without a kernel
 bool launch_hop_m5d(const HopM5dArgs& a, bool dag, hipStream_t st);
-bool hop_m5d_ok(int ls);
-int64_t hop_m5d_blocks(const LatGeo& g);
+// The vector updates of one FP64 CG iteration, with its scalars formed on
+// the device (Re <p, ap> in pap[0..npap), state st[slot]):
+//   k_cg_residual_d: alpha = |r|^2 / Re <p, ap>; r -= alpha ap; |r|^2 -> rnorm
+//   k_cg_step_d:     x += alpha p; unless converged p = r + beta p, t = Mat p;
+//                    the next iteration's state -> st[1 - slot] and *host
+struct CgIterDArgs {
+  LatGeo geo;
+  int ls;
+  const cplx<double>* mat;
+  bool real_mat;
+  double2 *x, *p, *r, *t;
+  const double2* ap;
+  const double* pap;
+  int npap;
+  double* rnorm;   // kMaxCgResidualGrid doubles
+  CgState64* st;   // [2]
+  int slot;
+  CgState64* host; // mapped host copy of the newest state
+};
+constexpr int kMaxCgResidualGrid = 512;
+void launch_cg_init_d(CgState64* st, double rr, double target, hipStream_t s);
+void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st);
+int64_t hop_m5d_blocks(const LatGeo& g, int ls);
 
 // r_i -= alpha_i ap_i with per-column partial |r_i|^2 (part[i*nblk + block])
 template <class S>
@@ -217,6 +250,8 @@ void launch_force(const ForceArgs& a, hipStream_t st);
 
 template <class T>
 void launch_hop(const HopArgs<T>& a, bool dag, int spt, hipStream_t st);
+// the FP64 hop (one column: cols ignored)
+void launch_hop_d(const HopArgs<double>& a, bool dag, hipStream_t st);
 // returns false (nothing launched) when ls is too large for the fused kernel
 bool launch_hop_m5(const HopM5Args& a, bool dag, hipStream_t st);
 int64_t hop_m5_blocks(const LatGeo& g);
@@ -318,6 +353,8 @@ void launch_h2d(const uint4* in, double2* out, int ls, int64_t n5, int acc, doub
 void launch_hop_h16(const HopArgs<float>& a, bool dag, hipStream_t st);
 template <class T>
 void launch_m5(const M5Args<T>& a, hipStream_t st);
+// the FP64 s-matrix (one column: cols ignored; no dotp)
+void launch_smat_d(const M5Args<double>& a, hipStream_t st);
 template <class T>
 void launch_cg_step(const CgStepArgs<T>& a, hipStream_t st);
 template <class S>

@@ -219,7 +219,6 @@ void launch_hop(const HopArgs<T>& a, bool dag, int spt, hipStream_t st)
   }
 }
 
-template void launch_hop<double>(const HopArgs<double>&, bool, int, hipStream_t);
 template void launch_hop<float>(const HopArgs<float>&, bool, int, hipStream_t);
 
 void launch_hop_h16(const HopArgs<float>& a, bool dag, hipStream_t st) { launch_hop_lds<Half16, 4, false>(a, dag, st); }
@@ -408,167 +407,6 @@ bool launch_hop_m5(const HopM5Args& a, bool dag, hipStream_t st)
   if (a.ls <= 8) launch_hop_m5_ls<kHopM5Sites, 8>(a, dag, st);
   else if (a.ls <= 12) launch_hop_m5_ls<kHopM5Sites, 12>(a, dag, st);
   else launch_hop_m5_ls<kHopM5Sites, 16>(a, dag, st);
-  return true;
-}
-
-// ================================================ FP64 hop + s-matrix
-// out = alpha * Mat (H in) + beta * x on FP64 fields (one column), in the
-// three phases of k_hop_m5s: a block is SB output half-sites x Ls rows;
-// phase 1, thread (site, s) forms the hop of its 5D site with the block's
-// links staged in LDS; phase 2, the Ls hop results of each site go through
-// LDS and thread (site, s) forms row s of the dense s-matrix product;
-// phase 3 adds beta * x, stores, and reduces Re <dotp, out> per block.
-// The links' LDS space is reused for the hop results once every thread
-// has finished phase 1.
-template <int SB, int LSMAX>
-__device__ __forceinline__ void stage_km_d(cplx<double> (*km)[LSMAX][LSMAX], const cplx<double>* __restrict__ M,
-                                           int ls)
-{
-  for (int i = threadIdx.x; i < 2 * LSMAX * LSMAX; i += blockDim.x) {
-    const int chi = i / (LSMAX * LSMAX), r = (i / LSMAX) % LSMAX, t = i % LSMAX;
-    if (r < ls && t < ls) km[chi][r][t] = M[(chi * ls + r) * ls + t];
-  }
-}
-
-template <int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT>
-__global__ void __launch_bounds__(SB * LSMAX) k_hop_m5d(HopM5dArgs a)
-{
-  constexpr int NSLOT = (72 > LSMAX * 12) ? 72 : LSMAX * 12;
-  __shared__ double2 buf[NSLOT][SB];  // links [72][SB], then hop results [LSMAX * 12][SB]
-  __shared__ int nbs[8][SB];
-  __shared__ cplx<double> km[2][LSMAX][LSMAX];
-  const unsigned lb = (unsigned)xcd_logical_block(blockIdx.x, (int64_t)gridDim.x);
-  const int64_t h0 = (int64_t)lb * SB;
-  const int pslot = (a.eo_out == 2) ? 0 : 1;
-  const double2* __restrict__ links = a.links + lidx(a.geo.stride, pslot, 0, h0);
-  for (int i = threadIdx.x; i < 72 * SB; i += blockDim.x) buf[i / SB][i % SB] = links[(i / SB) * 64 + (i % SB)];
-  for (int i = threadIdx.x; i < 8 * SB; i += blockDim.x) {  // thread (site, d): neighbour d
-    const int st = i % SB, d = i / SB;
-    if (h0 + st < a.geo.vh) nbs[d][st] = (int)neighbour_of(a.geo, h0 + st, a.eo_out, d);
-  }
-  stage_km_d<SB, LSMAX>(km, a.mat, a.ls);
-  __syncthreads();
-  const int ls = a.ls;
-  const int site = threadIdx.x % SB, row = threadIdx.x / SB;
-  const int64_t h = h0 + site;
-  const bool active = h < a.geo.vh && row < ls;
-  cplx<double> acc[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) acc[k] = cmk<double>(0, 0);
-  if (active) {
-    constexpr int SF = DAG ? 1 : -1;
-    constexpr int SG = -SF;
-#define QDWF_D(D, MU, SGN)                                         \
-  {                                                                \
-    cplx<double> W[9];                                             \
-    _Pragma("unroll") for (int e = 0; e < 9; ++e)                  \
-    {                                                              \
-      const double2 q = buf[(D) * 9 + e][site];                    \
-      W[e] = cmk<double>(q.x, q.y);                                \
-    }                                                              \
-    cplx<double> psi[12];                                          \
-    SpinorIO<double>::load(a.in, ls, row, nbs[D][site], psi);      \
-    hop_term<MU, SGN>(W, psi, acc);                                \
-  }
-    QDWF_D(0, 0, SF) QDWF_D(1, 1, SF) QDWF_D(2, 2, SF) QDWF_D(3, 3, SF)
-    QDWF_D(4, 0, SG) QDWF_D(5, 1, SG) QDWF_D(6, 2, SG) QDWF_D(7, 3, SG)
-#undef QDWF_D
-  }
-  const double sc = -0.5 * a.alpha;
-  __syncthreads();  // every thread is done with the links: buf becomes hr
-  double2 (*hr)[SB] = buf;  // hr[row * 12 + k][site]
-  if (active) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) hr[row * 12 + k][site] = make_double2(sc * acc[k].re, sc * acc[k].im);
-  }
-  __syncthreads();
-  double dot = 0.0;
-  if (active) {
-    cplx<double> v[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) v[k] = cmk<double>(0, 0);
-#pragma unroll
-    for (int t = 0; t < LSMAX; ++t) {
-      if (t < ls) {
-        const cplx<double> k0 = km[0][row][t], k1 = km[1][row][t];
-#pragma unroll
-        for (int k = 0; k < 12; ++k) {
-          const cplx<double> m = k < 6 ? k0 : k1;  // spins 0, 1: chirality 0
-          const double2 q = hr[t * 12 + k][site];
-          if (REAL) {
-            v[k].re += m.re * q.x;
-            v[k].im += m.re * q.y;
-          } else {
-            v[k] = cfma(v[k], m, cmk<double>(q.x, q.y));
-          }
-        }
-      }
-    }
-    if (XPAY) {
-      cplx<double> xv[12];
-      SpinorIO<double>::load(a.x, ls, row, h, xv);
-#pragma unroll
-      for (int k = 0; k < 12; ++k) v[k] = cmk<double>(v[k].re + a.beta * xv[k].re, v[k].im + a.beta * xv[k].im);
-    }
-    SpinorIO<double>::store_stream(a.out, ls, row, h, v);
-    if (DOT) {
-      cplx<double> pv[12];
-      SpinorIO<double>::load(a.dotp, ls, row, h, pv);
-#pragma unroll
-      for (int k = 0; k < 12; ++k) dot += pv[k].re * v[k].re + pv[k].im * v[k].im;
-    }
-  }
-  if (DOT) {
-    __shared__ double red[(SB * LSMAX + 63) / 64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) dot += __shfl_down(dot, o, 64);
-    if (lane == 0) red[wv] = dot;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double t = 0.0;
-      for (int i = 0; i < (int)((blockDim.x + 63) >> 6); ++i) t += red[i];
-      a.part[lb] = t;
-    }
-  }
-}
-
-template <int SB, int LSMAX>
-static void launch_hop_m5d_ls(const HopM5dArgs& a, bool dag, hipStream_t st)
-{
-  const dim3 grid((unsigned)((a.geo.vh + SB - 1) / SB));
-  const dim3 blk(SB * a.ls);
-  const bool xpay = a.x != nullptr, dot = a.dotp != nullptr;
-#define QDWF_L(D, X, R, DT) hipLaunchKernelGGL((k_hop_m5d<SB, LSMAX, D, X, R, DT>), grid, blk, 0, st, a)
-  if (dot) {
-    if (dag && xpay && a.real_mat) QDWF_L(true, true, true, true);
-    else if (dag && xpay) QDWF_L(true, true, false, true);
-    return;
-  }
-  if (a.real_mat) {
-    if (!dag && !xpay) QDWF_L(false, false, true, false);
-    if (!dag && xpay) QDWF_L(false, true, true, false);
-    if (dag && !xpay) QDWF_L(true, false, true, false);
-    if (dag && xpay) QDWF_L(true, true, true, false);
-  } else {
-    if (!dag && !xpay) QDWF_L(false, false, false, false);
-    if (!dag && xpay) QDWF_L(false, true, false, false);
-    if (dag && !xpay) QDWF_L(true, false, false, false);
-    if (dag && xpay) QDWF_L(true, true, false, false);
-  }
-#undef QDWF_L
-}
-
-bool hop_m5d_ok(int ls) { return ls >= 4 && ls <= 16 && (16 * ls) % 64 == 0; }
-int64_t hop_m5d_blocks(const LatGeo& g) { return (g.vh + 15) / 16; }
-
-bool launch_hop_m5d(const HopM5dArgs& a, bool dag, hipStream_t st)
-{
-  if (!hop_m5d_ok(a.ls) || !a.mat) return false;
-  if (a.dotp && !(dag && a.x)) return false;
-  if (a.ls <= 8) launch_hop_m5d_ls<16, 8>(a, dag, st);
-  else if (a.ls <= 12) launch_hop_m5d_ls<16, 12>(a, dag, st);
-  else launch_hop_m5d_ls<16, 16>(a, dag, st);
   return true;
 }
 
@@ -1532,7 +1370,6 @@ void launch_cg_step(const CgStepArgs<T>& a, hipStream_t st)
   else launch_cg_step_ls<T, 32>(a, st);
 }
 
-template void launch_cg_step<double>(const CgStepArgs<double>&, hipStream_t);
 template void launch_cg_step<float>(const CgStepArgs<float>&, hipStream_t);
 
 template <class T, int LSMAX>
@@ -1561,7 +1398,6 @@ void launch_m5(const M5Args<T>& a, hipStream_t st)
   else launch_m5_ls<T, 32>(a, st);
 }
 
-template void launch_m5<double>(const M5Args<double>&, hipStream_t);
 template void launch_m5<float>(const M5Args<float>&, hipStream_t);
 
 // ================================================================ BLAS-1
