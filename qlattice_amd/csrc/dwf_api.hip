@@ -162,6 +162,70 @@ enum Work64 {
 };
 enum Work32 { V_R, V_P, V_AP, V_X, V_T, V_T1, V_T2, V_T3, V_Y, W_COUNT32 };
 
+// A device-driven CG: the iteration's scalars live in two state slots on the
+// device (CgState64; an iteration reads slot it & 1 and writes the other),
+// and iterations are queued kCgAhead at a time, one group ahead of the group
+// the host waits for; those behind the converged one find its state and do
+// nothing.  No iteration waits for the host: 8^3x16 Ls8, 155 FP64 iterations
+// of 65 us, the solve 18.0 -> 10.7 ms with two host round trips less each.
+constexpr int kCgAhead = 2;
+constexpr int kRedDoubles = 4 * qdwf::kMaxRhs;  // reduction results of an inverter, its CG states behind them
+constexpr int64_t kMaxPrologueSums = 4096;  // more block sums go through a reduction kernel
+struct CgControl {
+  qdwf::CgState64* dev = nullptr;      // [2], the caller's
+  qdwf::CgState64* map = nullptr;      // mapped host copy of the newest state
+  qdwf::CgState64* map_dev = nullptr;
+  bool own_map = false;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  // map_host null: a mapped page of its own
+  CgControl(void* dev_states, void* map_host, void* map_device)
+      : dev((qdwf::CgState64*)dev_states), map((qdwf::CgState64*)map_host), map_dev((qdwf::CgState64*)map_device)
+  {
+    try {
+      if (!map) {
+        QDWF_HIP(hipHostMalloc((void**)&map, sizeof(qdwf::CgState64), hipHostMallocMapped | hipHostMallocCoherent));
+        own_map = true;
+        QDWF_HIP(hipHostGetDevicePointer((void**)&map_dev, map, 0));
+      }
+      for (auto& e : ev) QDWF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    } catch (...) {
+      release();
+      throw;
+    }
+  }
+  ~CgControl() { release(); }
+  CgControl(const CgControl&) = delete;
+  CgControl& operator=(const CgControl&) = delete;
+  void release()
+  {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (own_map && map) (void)hipHostFree(map);
+  }
+  // queue(slot) launches one iteration; returns the last state
+  template <class Queue>
+  qdwf::CgState64 run(double rr, double target, long max_num_iter, hipStream_t st, Queue&& queue)
+  {
+    *map = qdwf::CgState64{};
+    qdwf::launch_cg_init_d(dev, rr, target, st);
+    QDWF_HIP(hipGetLastError());
+    long queued = 0;
+    auto group = [&](hipEvent_t e) {
+      for (int j = 0; j < kCgAhead && queued < max_num_iter; ++j, ++queued) queue((int)(queued & 1));
+      QDWF_HIP(hipEventRecord(e, st));
+    };
+    group(ev[0]);
+    for (long g = 1;; ++g) {
+      const bool last = queued >= max_num_iter;
+      if (!last) group(ev[g & 1]);
+      QDWF_HIP(hipEventSynchronize(ev[(g - 1) & 1]));
+      if (last || *(volatile int*)&map->done) break;
+    }
+    QDWF_HIP(hipStreamSynchronize(st));  // the group queued behind
+    return *map;
+  }
+};
+
 // Tile width (columns per multi-RHS block) and sites per block of the
 // three-phase solver.
 struct TileChoice {
@@ -227,12 +291,7 @@ struct qlat_dwf_inverter {
   // Off by default: measured at most 2.5% faster (8^3x16) and 1-5% slower
   // from 12^3x24 up, where a host round trip is a small part of an iteration.
   int graph_iters = 0;
-  // FP64 CG: scalars of two iterations, their mapped host copy, the events
-  // of the two groups of iterations in flight
-  qdwf::CgState64* cg64 = nullptr;
-  qdwf::CgState64* cg64_map = nullptr;
-  qdwf::CgState64* cg64_map_dev = nullptr;
-  hipEvent_t cg64_ev[2] = {nullptr, nullptr};
+  std::unique_ptr<CgControl> cg64;  // of the FP64 CG, made at its first solve
   qdwf::CgState* cg_dev = nullptr;
   qdwf::CgState* cg_host = nullptr;
 
@@ -792,25 +851,11 @@ long cg_fp64(Inv& I, double2* x, const double2* b, double stop_rsd, long max_num
   m5<double>(I, t, p, MAT_K);
   const double qnorm_in = dev_norm2(I, b);
   const double qnorm_r = dev_norm2(I, r);
-  // The iteration's scalars stay on the device (dslash.h:365-392: alpha =
-  // |r|^2 / Re <p, A p>, r -= alpha A p, x += alpha p, beta, p = r + beta p),
-  // and iterations are queued kCgAhead at a time, one group ahead of the one
-  // the host waits for; those behind the converged one find its state and do
-  // nothing.  8^3x16 Ls8, whose iteration is 65 us of kernels: the solve
-  // 18.0 -> 10.7 ms.
-  constexpr int kCgAhead = 2;
-  if (!I.cg64) {
-    I.cg64 = (qdwf::CgState64*)dev_alloc(2 * sizeof(qdwf::CgState64));
-    QDWF_HIP(hipHostMalloc((void**)&I.cg64_map, sizeof(qdwf::CgState64), hipHostMallocMapped | hipHostMallocCoherent));
-    QDWF_HIP(hipHostGetDevicePointer((void**)&I.cg64_map_dev, I.cg64_map, 0));
-    for (auto& e : I.cg64_ev) QDWF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
-  *I.cg64_map = qdwf::CgState64{};
-  qdwf::launch_cg_init_d(I.cg64, qnorm_r, qnorm_in * stop_rsd * stop_rsd, I.stream);
-  check_launch();
-  // sums of many blocks go through a reduction kernel first
+  // alpha = |r|^2 / Re <p, A p>, r -= alpha A p, x += alpha p, beta,
+  // p = r + beta p (dslash.h:365-392) and t = K p, the scalars on the device
+  if (!I.cg64) I.cg64.reset(new CgControl(I.red + kRedDoubles, I.red_map + kRedDoubles, I.red_map_dev + kRedDoubles));
   const int64_t nblk = qdwf::hop_m5d_blocks(I.geo, I.ls);
-  const bool reduce = nblk > 4096;
+  const bool reduce = nblk > kMaxPrologueSums;
   qdwf::CgIterDArgs ia{};
   ia.geo = I.geo;
   ia.ls = I.ls;
@@ -824,33 +869,19 @@ long cg_fp64(Inv& I, double2* x, const double2* b, double stop_rsd, long max_num
   ia.pap = reduce ? I.red : I.part;
   ia.npap = reduce ? 1 : (int)nblk;
   ia.rnorm = I.part + nblk;
-  ia.st = I.cg64;
-  ia.host = I.cg64_map_dev;
-  long queued = 0;
-  auto queue_group = [&](hipEvent_t ev) {
-    for (int j = 0; j < kCgAhead && queued < max_num_iter; ++j, ++queued) {
-      ia.slot = (int)(queued & 1);
-      hermop_t1_dot64(I, ap, p, t, 1, I.cg64 + ia.slot);
-      if (reduce) qdwf::launch_reduce_rows(I.part, (int)nblk, 1, I.red, I.stream);
-      qdwf::launch_cg_iter_d(ia, I.stream);
-      check_launch();
-    }
-    QDWF_HIP(hipEventRecord(ev, I.stream));
-  };
-  queue_group(I.cg64_ev[0]);
-  for (long g = 1;; ++g) {
-    const bool last = queued >= max_num_iter;
-    if (!last) queue_group(I.cg64_ev[g & 1]);
-    QDWF_HIP(hipEventSynchronize(I.cg64_ev[(g - 1) & 1]));
-    if (*(volatile int*)&I.cg64_map->done || last) {
-      sync(I);  // the groups queued behind
-      const qdwf::CgState64 end = *I.cg64_map;
-      I.stats.hermop_fp64 += end.iter;
-      if (end.done == 2) throw std::runtime_error("CG breakdown: non-finite residual (FP64)");
-      if (end.done) return (long)end.iter;
-      break;
-    }
-  }
+  ia.st = I.cg64->dev;
+  ia.host = I.cg64->map_dev;
+  const qdwf::CgState64 end =
+      I.cg64->run(qnorm_r, qnorm_in * stop_rsd * stop_rsd, max_num_iter, I.stream, [&](int slot) {
+        ia.slot = slot;
+        hermop_t1_dot64(I, ap, p, t, 1, I.cg64->dev + slot);
+        if (reduce) qdwf::launch_reduce_rows(I.part, (int)nblk, 1, I.red, I.stream);
+        qdwf::launch_cg_iter_d(ia, I.stream);
+        check_launch();
+      });
+  I.stats.hermop_fp64 += end.iter;
+  if (end.done == 2) throw std::runtime_error("CG breakdown: non-finite residual (FP64)");
+  if (end.done) return (long)end.iter;
   return max_num_iter + 1;
 }
 
@@ -2454,10 +2485,6 @@ void free_all(Inv* I)
   f(I->part);
   f(I->red);
   if (I->red_map) (void)hipHostFree(I->red_map);
-  f(I->cg64);
-  if (I->cg64_map) (void)hipHostFree(I->cg64_map);
-  for (auto e : I->cg64_ev)
-    if (e) (void)hipEventDestroy(e);
   f(I->cg_dev);
   if (I->cg_host) (void)hipHostFree(I->cg_host);
   f(I->lm_basis);
@@ -2592,9 +2619,9 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
       I->part_cap = np * qdwf::kMaxRhs;
       I->part = (double*)dev_alloc(I->part_cap * sizeof(double));
     }
-    I->red = (double*)dev_alloc(4 * qdwf::kMaxRhs * sizeof(double));
-    QDWF_HIP(hipHostMalloc((void**)&I->red_map, 4 * qdwf::kMaxRhs * sizeof(double),
-                           hipHostMallocMapped | hipHostMallocCoherent));
+    const size_t rbytes = kRedDoubles * sizeof(double) + 2 * sizeof(qdwf::CgState64);
+    I->red = (double*)dev_alloc(rbytes);
+    QDWF_HIP(hipHostMalloc((void**)&I->red_map, rbytes, hipHostMallocMapped | hipHostMallocCoherent));
     QDWF_HIP(hipHostGetDevicePointer((void**)&I->red_map_dev, I->red_map, 0));
     *out = I;
   });
@@ -3012,27 +3039,54 @@ struct QedCall {
     for (int mu = 0; mu < 4; ++mu) {
       QDWF_REQUIRE(total_site[mu] > 0, "total_site must be positive");
       a.n[mu] = total_site[mu];
+      if (mu < 3) a.dn[mu] = qdwf::make_fastdiv((unsigned)total_site[mu]);
       vol *= total_site[mu];
     }
     n = vol * ls * 4;
     a.ls = ls;
+    a.nelem = n;
+    a.dls = qdwf::make_fastdiv((unsigned)ls);
     a.mass = mass;
     a.m5 = m5;
-    gf.reset(new DevBuf(vol * 4 * sizeof(double2)));
-    QDWF_HIP(hipMemcpy(gf->p, gf1, vol * 4 * sizeof(double2), hipMemcpyHostToDevice));
+    const size_t gbytes = vol * 4 * sizeof(double2);
+    gf.reset(new DevBuf(2 * gbytes));
+    QDWF_HIP(hipMemcpy(gf->p, gf1, gbytes, hipMemcpyHostToDevice));
+    qdwf::launch_qed_inverse(gf->d(), gf->d() + vol * 4, vol * 4, nullptr);
+    check_launch();
     a.gf = gf->d();
+    a.gfi = gf->d() + vol * 4;
     if (wick_h) {
-      wick.reset(new DevBuf(total_site[3] * sizeof(double2)));
-      QDWF_HIP(hipMemcpy(wick->p, wick_h, total_site[3] * sizeof(double2), hipMemcpyHostToDevice));
+      // the time slices' averages and inverses (qed.cpp:312-328)
+      const int T = total_site[3];
+      std::vector<cd> w((size_t)T * 4);
+      auto at = [&](int t) { return cd(wick_h[2 * t], wick_h[2 * t + 1]); };
+      auto inverse = [](cd z) {
+        const double d = z.real() * z.real() + z.imag() * z.imag();
+        return cd(z.real() / d, -z.imag() / d);
+      };
+      for (int t = 0; t < T; ++t) {
+        const cd tw = at(t), twm = at((t - 1 + T) % T);
+        const cd itw = inverse(tw), itwm = inverse(twm);
+        w[4 * t] = 0.5 * tw + 0.5 * twm;
+        w[4 * t + 1] = 0.5 * itw + 0.5 * itwm;
+        w[4 * t + 2] = itw;
+        w[4 * t + 3] = itwm;
+      }
+      wick.reset(new DevBuf(w.size() * sizeof(cd)));
+      QDWF_HIP(hipMemcpy(wick->p, w.data(), w.size() * sizeof(cd), hipMemcpyHostToDevice));
       a.wick = wick->d();
     }
   }
-  void apply(double2* out, const double2* in, bool dagger) const
+  void apply(double2* out, const double2* in, bool dagger, const double2* dotp = nullptr, double* part = nullptr,
+             const qdwf::CgState64* cg = nullptr) const
   {
     qdwf::QedArgs b = a;
     b.in = in;
     b.out = out;
     b.dagger = dagger ? 1 : 0;
+    b.dotp = dotp;
+    b.part = part;
+    b.cg = cg;
     qdwf::launch_qed_m(b, nullptr);
     check_launch();
   }
@@ -3046,41 +3100,52 @@ double qed_norm2(const double2* x, int64_t n, double* part, double* red)
   return v;
 }
 
-// cg_with_m_dwf_qed (qed.cpp:178-261): M_{!d} M_{d} x = b from the guess in x
+// cg_with_m_dwf_qed (qed.cpp:178-261): M_{!d} M_{d} x = b from the guess in
+// x, with the scalars on the device and the iterations queued ahead as in
+// cg_fp64
 long qed_cg(const QedCall& q, double2* x, const double2* b, bool dagger, double stop_rsd, long max_num_iter)
 {
   QDWF_REQUIRE(stop_rsd >= 0.0 && max_num_iter >= 0, "invalid stop_rsd or max_num_iter");
   if (max_num_iter == 0) return 0;
   const int64_t n = q.n;
   const size_t fb = n * sizeof(double2);
-  DevBuf r(fb), p(fb), ap(fb), tmp(fb), part(2 * qdwf::kMaxBlasGrid * sizeof(double)), red(2 * sizeof(double));
-  auto A = [&](double2* out, const double2* in) {
-    q.apply(tmp.d(), in, dagger);
-    q.apply(out, tmp.d(), !dagger);
-  };
-  QDWF_HIP(hipMemcpy(r.p, b, fb, hipMemcpyDeviceToDevice));
-  A(ap.d(), x);
-  qdwf::launch_axpy<double2>(-1.0, ap.d(), r.d(), n, nullptr);
+  const int64_t nblk = qdwf::qed_m_blocks(q.a);
+  const int64_t nparts = std::max<int64_t>(nblk + qdwf::kMaxCgResidualGrid, 2 * qdwf::kMaxBlasGrid);
+  // r, p, ap, tmp, the partial sums, two reduction results, two CG states
+  const size_t tail = (nparts + 2) * sizeof(double) + 2 * sizeof(qdwf::CgState64);
+  DevBuf buf(4 * fb + tail);
+  double2 *r = buf.d(), *pv = r + n, *ap = pv + n, *tmp = ap + n;
+  double *part = (double*)(tmp + n), *red = part + nparts;
+  CgControl ctl(red + 2, nullptr, nullptr);
+  QDWF_HIP(hipMemcpyAsync(r, b, fb, hipMemcpyDeviceToDevice, nullptr));
+  q.apply(tmp, x, dagger);
+  q.apply(ap, tmp, !dagger);
+  qdwf::launch_axpy<double2>(-1.0, ap, r, n, nullptr);
   check_launch();
-  QDWF_HIP(hipMemcpy(p.p, r.p, fb, hipMemcpyDeviceToDevice));
-  const double qnorm_in = qed_norm2(b, n, (double*)part.p, (double*)red.p);
-  double qnorm_r = qed_norm2(r.d(), n, (double*)part.p, (double*)red.p);
-  for (long iter = 1; iter <= max_num_iter; ++iter) {
-    A(ap.d(), p.d());
-    qdwf::launch_dot<double2>(p.d(), ap.d(), n, (double*)part.p, (double*)red.p, nullptr);
-    double pap[2];
-    QDWF_HIP(hipMemcpy(pap, red.p, 2 * sizeof(double), hipMemcpyDeviceToHost));
-    const double alpha = qnorm_r / pap[0];
-    qdwf::launch_axpy<double2>(alpha, p.d(), x, n, nullptr);
-    qdwf::launch_axpy<double2>(-alpha, ap.d(), r.d(), n, nullptr);
+  QDWF_HIP(hipMemcpyAsync(pv, r, fb, hipMemcpyDeviceToDevice, nullptr));
+  const double qnorm_in = qed_norm2(b, n, part, red);
+  const double qnorm_r = qed_norm2(r, n, part, red);
+  const bool reduce = nblk > kMaxPrologueSums;
+  qdwf::QedIterArgs ia{};
+  ia.n = n;
+  ia.x = x;
+  ia.p = pv;
+  ia.r = r;
+  ia.ap = ap;
+  ia.pap = reduce ? red : part;
+  ia.npap = reduce ? 1 : (int)nblk;
+  ia.rnorm = part + nblk;
+  ia.st = ctl.dev;
+  ia.host = ctl.map_dev;
+  const qdwf::CgState64 end = ctl.run(qnorm_r, qnorm_in * stop_rsd * stop_rsd, max_num_iter, nullptr, [&](int slot) {
+    ia.slot = slot;
+    q.apply(tmp, pv, dagger, nullptr, nullptr, ctl.dev + slot);
+    q.apply(ap, tmp, !dagger, pv, part, ctl.dev + slot);
+    if (reduce) qdwf::launch_reduce_rows(part, (int)nblk, 1, red, nullptr);
+    qdwf::launch_qed_iter(ia, nullptr);
     check_launch();
-    const double new_qnorm_r = qed_norm2(r.d(), n, (double*)part.p, (double*)red.p);
-    if (new_qnorm_r <= qnorm_in * stop_rsd * stop_rsd) return iter;
-    qdwf::launch_xpay<double2>(r.d(), new_qnorm_r / qnorm_r, p.d(), n, nullptr);  // p = r + beta p
-    check_launch();
-    qnorm_r = new_qnorm_r;
-  }
-  return max_num_iter + 1;
+  });
+  return end.done ? (long)end.iter : max_num_iter + 1;
 }
 
 }  // namespace
@@ -3207,29 +3272,17 @@ int qlat_dwf_invert_dwf_qed(const int total_site[4], int ls, const double* gf1, 
     const QedCall q(total_site, ls, gf1, mass, m5, wick);
     const int64_t vol = q.vol;
     const size_t fb = q.n * sizeof(double2);
-    // fermion_field_5d_from_4d_qed(src5d, in, ls, 0, ls - 1) on the host side of the copy
-    std::vector<double2> h5((size_t)q.n, make_double2(0.0, 0.0));
-    const double2* in = (const double2*)in4d;
-    for (int64_t x = 0; x < vol; ++x) {
-      h5[(x * ls + 0) * 4 + 0] = in[x * 4 + 0];
-      h5[(x * ls + 0) * 4 + 1] = in[x * 4 + 1];
-      h5[(x * ls + ls - 1) * 4 + 2] = in[x * 4 + 2];
-      h5[(x * ls + ls - 1) * 4 + 3] = in[x * 4 + 3];
-    }
-    DevBuf s5(fb), b5(fb), x5(fb);
-    QDWF_HIP(hipMemcpy(s5.p, h5.data(), fb, hipMemcpyHostToDevice));
+    DevBuf f4(vol * 4 * sizeof(double2)), s5(fb), b5(fb);
+    QDWF_HIP(hipMemcpy(f4.p, in4d, vol * 4 * sizeof(double2), hipMemcpyHostToDevice));
+    qdwf::launch_qed_embed(f4.d(), s5.d(), ls, vol, nullptr);
+    check_launch();
     q.apply(b5.d(), s5.d(), is_dagger == 0);  // M_{!d} src (qed.cpp:141-142)
-    QDWF_HIP(hipMemset(x5.p, 0, fb));
-    *iter = qed_cg(q, x5.d(), b5.d(), is_dagger != 0, stop_rsd, max_num_iter);
-    QDWF_HIP(hipMemcpy(h5.data(), x5.p, fb, hipMemcpyDeviceToHost));
-    // fermion_field_4d_from_5d_qed(out, sol5d, ls, ls - 1, 0)
-    double2* out = (double2*)out4d;
-    for (int64_t x = 0; x < vol; ++x) {
-      out[x * 4 + 0] = h5[(x * ls + ls - 1) * 4 + 0];
-      out[x * 4 + 1] = h5[(x * ls + ls - 1) * 4 + 1];
-      out[x * 4 + 2] = h5[(x * ls + 0) * 4 + 2];
-      out[x * 4 + 3] = h5[(x * ls + 0) * 4 + 3];
-    }
+    double2* x5 = s5.d();                     // (the 5D source is not needed any more)
+    QDWF_HIP(hipMemsetAsync(x5, 0, fb, nullptr));
+    *iter = qed_cg(q, x5, b5.d(), is_dagger != 0, stop_rsd, max_num_iter);
+    qdwf::launch_qed_project(x5, f4.d(), ls, vol, nullptr);
+    check_launch();
+    QDWF_HIP(hipMemcpy(out4d, f4.p, vol * 4 * sizeof(double2), hipMemcpyDeviceToHost));
   });
 }
 

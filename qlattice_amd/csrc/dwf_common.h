@@ -758,4 +758,28 @@ __device__ __forceinline__ void hop_term_h2(const h16x2 la[9], const h16x2 lb[9]
   }
 }
 
+// Sum of v over the block (up to MAXW waves); every thread gets it.
+template <int MAXW>
+__device__ __forceinline__ double block_sum(double v)
+{
+  __shared__ double red[MAXW];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  if (lane == 0) red[wv] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int i = 0; i < nw; ++i) t += red[i];
+  return t;
+}
+
+// The sum of n partial sums in every block of 256 threads, always in the same
+// order (the prologue of kernels that use the previous kernel's block sums).
+__device__ __forceinline__ double sum_parts(const double* __restrict__ part, int n)
+{
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) v += part[i];
+  return block_sum<4>(v);
+}
+
 }  // namespace qdwf

@@ -58,21 +58,6 @@ struct SMat {
   }
 };
 
-// Sum of v over the block (up to MAXW waves); every thread gets it.
-template <int MAXW>
-__device__ __forceinline__ double block_sum(double v)
-{
-  __shared__ double red[MAXW];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  if (lane == 0) red[wv] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int i = 0; i < nw; ++i) t += red[i];
-  return t;
-}
-
 // out = alpha Mat in (+ beta x): wave = 16 sites x kSmatComps components of
 // one chirality, block = 64 sites, blockIdx.y = the component group.
 // HBM bound, at the speed of a copy: 0.43 ms at 24^3x64 Ls12 (4.7 TB/s),
@@ -175,13 +160,6 @@ void launch_cg_init_d(CgState64* st, double rr, double target, hipStream_t s)
   hipLaunchKernelGGL(k_cg_init_d, dim3(1), dim3(1), 0, s, st, rr, target);
 }
 
-__device__ __forceinline__ double sum_parts(const double* __restrict__ part, int n)
-{
-  double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) v += part[i];
-  return block_sum<4>(v);
-}
-
 __global__ void __launch_bounds__(256) k_cg_residual_d(CgIterDArgs a, int64_t n)
 {
   CgState64* st = a.st + a.slot;
@@ -280,7 +258,7 @@ static void launch_cg_step_d_ls(const CgIterDArgs& a, int nrnorm, hipStream_t st
 void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st)
 {
   const int64_t n = (int64_t)a.ls * 12 * a.geo.stride;
-  const int g = (int)((n + 1023) / 1024 < kMaxCgResidualGrid ? (n + 1023) / 1024 : kMaxCgResidualGrid);
+  const int g = cg_residual_grid(n);
   hipLaunchKernelGGL(k_cg_residual_d, dim3(g), dim3(256), 0, st, a, n);
   if (a.ls <= 8) launch_cg_step_d_ls<8>(a, g, st);
   else if (a.ls <= 12) launch_cg_step_d_ls<12>(a, g, st);

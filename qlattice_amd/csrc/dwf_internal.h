@@ -206,6 +206,10 @@ struct CgIterDArgs {
   CgState64* host; // mapped host copy of the newest state
 };
 constexpr int kMaxCgResidualGrid = 512;
+inline int cg_residual_grid(int64_t n)
+{
+  return (int)((n + 1023) / 1024 < kMaxCgResidualGrid ? (n + 1023) / 1024 : kMaxCgResidualGrid);
+}
 void launch_cg_init_d(CgState64* st, double rr, double target, hipStream_t s);
 void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st);
 int64_t hop_m5d_blocks(const LatGeo& g, int ls);
@@ -284,13 +288,37 @@ void launch_make_src(double2* prop, const SrcArgs& a, hipStream_t st);
 struct QedArgs {
   int n[4];
   int ls;
+  int64_t nelem;        // V * ls * 4
+  FastDiv dls, dn[3];   // divisions by ls and X, Y, Z
   double mass, m5;
   const double2* gf;
-  const double2* wick;  // [T] or null
+  const double2* gfi;   // 1 / gf
+  const double2* wick;  // [T][4] or null: (tw + twm)/2, (1/tw + 1/twm)/2, 1/tw, 1/twm; twm = tw(t - 1)
   int dagger;
   const double2* in;
   double2* out;
+  const double2* dotp;  // optional: part[block] = Re <dotp, out>, qed_m_blocks of them
+  double* part;
+  const CgState64* cg;  // optional: nothing is done once cg->done
 };
+int64_t qed_m_blocks(const QedArgs& a);
+void launch_qed_inverse(const double2* gf, double2* inv, int64_t n, hipStream_t st);
+void launch_qed_embed(const double2* in4, double2* out5, int ls, int64_t vol, hipStream_t st);
+void launch_qed_project(const double2* in5, double2* out4, int ls, int64_t vol, hipStream_t st);
+// one CG iteration's vector updates (Re <p, ap> in pap[0..npap)): x += alpha
+// p, r -= alpha ap; p = r + beta p, state st[slot] -> st[1 - slot] and *host
+struct QedIterArgs {
+  int64_t n;  // elements
+  double2 *x, *p, *r;
+  const double2* ap;
+  const double* pap;
+  int npap;
+  double* rnorm;  // kMaxCgResidualGrid doubles
+  CgState64* st;
+  int slot;
+  CgState64* host;
+};
+void launch_qed_iter(const QedIterArgs& a, hipStream_t st);
 void launch_qed_m(const QedArgs& a, hipStream_t st);
 
 // Free-field domain-wall propagator (free_invert, qcd-prop.h:292-359) on
