@@ -2544,9 +2544,12 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
     I->geo.xh = total_site[0] / 2;
     // device site order: tiles of `by` rows in y and `bz` planes in z, each
     // swept in t (dwf_common.h); by = Y, bz = Z is the reference order.
-    // Defaults (measured at 24^3x64): by = the divisor of Y closest to 6,
-    // bz = Z (z tiles cut L2 misses of the FP16 hop by 20% without making
-    // it faster, and slow the FP32/FP64 hops by ~7%).
+    // Defaults: by = the divisor of Y closest to 6, bz = the divisor of Z
+    // closest to 8: a t step is then short enough for the L2 to keep the
+    // neighbouring time slices.  Mpc^+ Mpc at 24^3x64 Ls12, bz = 24 against
+    // 12 and 6: FP64 4.21, 3.90, 3.83 ms, FP32 2.01, 1.89, 1.92 ms, FP16
+    // storage (12 columns, per column) 1.24, 1.12, 1.13 ms; 16^3x32 Ls12,
+    // bz = 16 against 8: 585, 554 us (FP64).
     // QLAT_DWF_TILE_Y / QLAT_DWF_TILE_Z override the defaults.
     auto tile_of = [](int n, int pref, const char* env) {
       int b = n;
@@ -2559,7 +2562,7 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
       return b;
     };
     I->geo.by = tile_of(total_site[1], 6, "QLAT_DWF_TILE_Y");
-    I->geo.bz = tile_of(total_site[2], total_site[2], "QLAT_DWF_TILE_Z");
+    I->geo.bz = tile_of(total_site[2], 8, "QLAT_DWF_TILE_Z");
     I->geo.vh = V / 2;
     I->geo.stride = (I->geo.vh + qdwf::kStrideAlign - 1) / qdwf::kStrideAlign * qdwf::kStrideAlign;
     I->geo.dxh = qdwf::make_fastdiv((unsigned)I->geo.xh);
