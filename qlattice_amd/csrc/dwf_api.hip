@@ -263,6 +263,7 @@ struct qlat_dwf_inverter {
   double2* l64 = nullptr;
   float2* l32 = nullptr;
   unsigned* l16 = nullptr;  // FP16 links for the FP16-arithmetic hop (h2_hop)
+  unsigned* nbt = nullptr;  // neighbour table of the three-phase kernels
   // FP16-storage solver: hop phase in FP16 arithmetic (FP16 links, packed
   // FP16 projection, v_dot2_f32_f16 SU(3) rows; QLAT_DWF_H2=0 selects FP32
   // arithmetic).  Measured at 24^3x64 Ls12, b = K H t over 4 columns:
@@ -1353,6 +1354,7 @@ struct ThreePhase {
     a.x = x;
     a.links = I.l32;
     a.links16 = half() ? I.l16 : nullptr;
+    a.nbt = I.nbt;
     a.hop_mode = I.h2_hop;
     a.plain64 = I.plain64;
     a.sb = sb;
@@ -2472,6 +2474,7 @@ void free_all(Inv* I)
   f(I->l64);
   f(I->l32);
   f(I->l16);
+  f(I->nbt);
   f(I->mat64);
   f(I->mat32);
   f(I->beta64);
@@ -2591,6 +2594,9 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
     double2* g = (double2*)dev_alloc(gbytes);
     QDWF_HIP(hipMemcpyAsync(g, gauge, gbytes, hipMemcpyHostToDevice, I->stream));
     pack_gauge_dev(*I, g);
+    I->nbt = (unsigned*)dev_alloc((size_t)16 * I->geo.stride * sizeof(unsigned));
+    qdwf::launch_neighbours(I->nbt, I->geo, I->stream);
+    check_launch();
     QDWF_HIP(hipStreamSynchronize(I->stream));
     QDWF_HIP(hipFree(g));
     build_matrices(*I);

@@ -213,6 +213,13 @@ __device__ __forceinline__ int64_t xcd_logical_block(int64_t b, int64_t nblk)
   return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// the same for block numbers below 2^32
+__device__ __forceinline__ unsigned xcd_logical_block32(unsigned b, unsigned nblk)
+{
+  const unsigned q = nblk >> 3, r = nblk & 7u, xcd = b & 7u, local = b >> 3;
+  return xcd * q + (xcd < r ? xcd : r) + local;
+}
+
 // Element i of a small by-value array (kernel arguments) without dynamic
 // indexing, which would copy the array to scratch memory; i is wave-uniform.
 template <class V, int N>
@@ -338,13 +345,39 @@ struct SpinorIO<float> {
       v[2 * k + 1] = cmk<float>(a.z, a.w);
     }
   }
+  // v += beta * f(s, h)
+  __device__ __forceinline__ static void fma_stream(const float4* __restrict__ f, int ls, int s, int64_t h, float beta,
+                                                    cplx<float> v[12])
+  {
+    cplx<float> x[12];
+    load_stream(f, ls, s, h, x);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) v[k] = cmk<float>(v[k].re + beta * x[k].re, v[k].im + beta * x[k].im);
+  }
+  // Re <f(s, h), v>
+  __device__ __forceinline__ static double dot_stream(const float4* __restrict__ f, int ls, int s, int64_t h,
+                                                      const cplx<float> v[12])
+  {
+    cplx<float> x[12];
+    load_stream(f, ls, s, h, x);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      t = fma((double)x[k].re, (double)v[k].re, t);
+      t = fma((double)x[k].im, (double)v[k].im, t);
+    }
+    return t;
+  }
   // raw loads (issued together, decoded later: more loads in flight per wave)
+  // from a site's place At, formed once for all its rows
   struct Raw {
     float4 q[6];
   };
-  __device__ __forceinline__ static void load_raw(const float4* __restrict__ f, int ls, int s, int64_t h, Raw& r)
+  typedef unsigned At;  // slot of row 0
+  __device__ __forceinline__ static At at(int ls, unsigned h) { return sidx<6>(ls, 0, 0, h); }
+  __device__ __forceinline__ static void load_raw(const float4* __restrict__ f, At a, int s, Raw& r)
   {
-    const float4* p = f + sidx<6>(ls, s, 0, h);
+    const float4* p = f + (a + (unsigned)s * 384u);
 #pragma unroll
     for (int k = 0; k < 6; ++k) r.q[k] = p[k * 64];
   }
@@ -381,6 +414,16 @@ __device__ __forceinline__ cplx<float> unpack_h2(unsigned w, float sc)
 {
   const h16x2 v = __builtin_bit_cast(h16x2, w);
   return cmk<float>((float)v.x * sc, (float)v.y * sc);
+}
+
+// max(|a|, |b|, m) as one v_max3_f32 (an ALU instruction only); fmaxf of
+// absolute values is compiled to canonicalising moves as well, 42 against 12
+// instructions for a site
+__device__ __forceinline__ float absmax3(float a, float b, float m)
+{
+  float r;
+  asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
+  return r;
 }
 
 template <>
@@ -426,12 +469,21 @@ struct SpinorIO<Half16> {
   {
     return (float*)((char*)f + byte);
   }
-  __device__ __forceinline__ static void load_raw(const uint4* __restrict__ f, int ls, int s, int64_t h, Raw& r)
+  // a site's place, formed once for all its rows: bytes of unit 0 and of the
+  // scale of row 0
+  struct At {
+    unsigned unit, scale;
+  };
+  __device__ __forceinline__ static At at(int ls, unsigned h)
   {
-    const unsigned b = base(ls, s, h), lane = (unsigned)h & 63u;
-    r.sc = *scale_at(f, scale_byte(ls, s, h));
+    return At{(base(ls, 0, h) + (h & 63u)) * 16u, scale_byte(ls, 0, h)};
+  }
+  __device__ __forceinline__ static void load_raw(const uint4* __restrict__ f, At a, int s, Raw& r)
+  {
+    r.sc = *scale_at(f, a.scale + ((unsigned)s << 6));
+    const unsigned b = a.unit + (unsigned)s * 3072u;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) r.q[j] = *slot_at(f, b + j * 64u + lane);
+    for (int j = 0; j < 3; ++j) r.q[j] = *(const uint4*)((const char*)f + b + j * 1024u);
   }
   __device__ __forceinline__ static void decode(const Raw& r, cplx<float> v[12])
   {
@@ -472,15 +524,57 @@ struct SpinorIO<Half16> {
       v[4 * j + 3] = unpack_h2(q.w, sc);
     }
   }
+  // v += beta * f(s, h)
+  __device__ __forceinline__ static void fma_stream(const uint4* __restrict__ f, int ls, int s, int64_t h, float beta,
+                                                    cplx<float> v[12])
+  {
+    const unsigned b = base(ls, s, h), lane = (unsigned)h & 63u;
+    const float bs = beta * __builtin_nontemporal_load(scale_at(f, scale_byte(ls, s, h)));
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const u32x4 q = __builtin_nontemporal_load((const u32x4*)slot_at(f, b + j * 64u + lane));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned u = q[i];  // (a bit cast of a vector's element takes element 0)
+        const h16x2 w = __builtin_bit_cast(h16x2, u);
+        v[4 * j + i].re = fmaf((float)w.x, bs, v[4 * j + i].re);
+        v[4 * j + i].im = fmaf((float)w.y, bs, v[4 * j + i].im);
+      }
+    }
+  }
+  // Re <f(s, h), v>
+  __device__ __forceinline__ static double dot_stream(const uint4* __restrict__ f, int ls, int s, int64_t h,
+                                                      const cplx<float> v[12])
+  {
+    const unsigned b = base(ls, s, h), lane = (unsigned)h & 63u;
+    const float sc = __builtin_nontemporal_load(scale_at(f, scale_byte(ls, s, h)));
+    double t = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const u32x4 q = __builtin_nontemporal_load((const u32x4*)slot_at(f, b + j * 64u + lane));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned u = q[i];  // (a bit cast of a vector's element takes element 0)
+        const h16x2 w = __builtin_bit_cast(h16x2, u);
+        t = fma((double)(float)w.x, (double)v[4 * j + i].re, t);
+        t = fma((double)(float)w.y, (double)v[4 * j + i].im, t);
+      }
+    }
+    return (double)sc * t;
+  }
+  // The scale is the power of two at or below the site's largest component,
+  // so that scaling is exact both ways (stored values stay below 2, 4 where
+  // the scale is capped).
   template <bool NT>
   __device__ __forceinline__ static void put(uint4* __restrict__ f, int ls, int s, int64_t h, cplx<float> v[12])
   {
     float m = 0.f;
 #pragma unroll
-    for (int k = 0; k < 12; ++k) m = fmaxf(m, fmaxf(fabsf(v[k].re), fabsf(v[k].im)));
-    // sites below 2^-100 are stored as zero: 1/m must stay finite
-    if (m < 0x1p-100f) m = 0.f;
-    const float inv = m > 0.f ? 1.f / m : 0.f;
+    for (int k = 0; k < 12; ++k) m = absmax3(v[k].re, v[k].im, m);
+    // sites below 2^-100 are stored as zero; the cap keeps 1/m normal
+    const unsigned e = min(__float_as_uint(m) & 0x7f800000u, 0x7e800000u);
+    m = m < 0x1p-100f ? 0.f : __uint_as_float(e);
+    const float inv = m > 0.f ? __uint_as_float(0x7f000000u - e) : 0.f;
     const unsigned b = base(ls, s, h), lane = (unsigned)h & 63u;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -728,8 +822,9 @@ __device__ __forceinline__ float fdot2_z(h16x2 a, h16x2 b)
   return r;
 }
 
-// acc += sc * (1 + sg gamma_mu) U psi with psi, U in FP16 (la, lb as above)
-template <int MU, int SG>
+// acc += sc * (1 + sg gamma_mu) U psi with psi, U in FP16 (la, lb as above);
+// FIRST: acc = (no sum with zeros)
+template <int MU, int SG, bool FIRST>
 __device__ __forceinline__ void hop_term_h2(const h16x2 la[9], const h16x2 lb[9], const h16x2 psi[12], float sc,
                                             cplx<float> acc[12])
 {
@@ -749,12 +844,19 @@ __device__ __forceinline__ void hop_term_h2(const h16x2 la[9], const h16x2 lb[9]
       y1i = __builtin_amdgcn_fdot2(lb[r * 3 + c], w1[c], y1i, false);
     }
     const cplx<float> y0 = cmk<float>(y0r, y0i), y1 = cmk<float>(y1r, y1i);
-    cfma_s(acc[r], sc, y0);
-    cfma_s(acc[3 + r], sc, y1);
     cplx<float> t2, t3;
     bdag<MU>(y0, y1, t2, t3);
-    cfma_s(acc[6 + r], ssg, t2);
-    cfma_s(acc[9 + r], ssg, t3);
+    if (FIRST) {
+      acc[r] = cmk<float>(sc * y0.re, sc * y0.im);
+      acc[3 + r] = cmk<float>(sc * y1.re, sc * y1.im);
+      acc[6 + r] = cmk<float>(ssg * t2.re, ssg * t2.im);
+      acc[9 + r] = cmk<float>(ssg * t3.re, ssg * t3.im);
+    } else {
+      cfma_s(acc[r], sc, y0);
+      cfma_s(acc[3 + r], sc, y1);
+      cfma_s(acc[6 + r], ssg, t2);
+      cfma_s(acc[9 + r], ssg, t3);
+    }
   }
 }
 

@@ -154,6 +154,9 @@ struct HopM5Args {
   int site_major;
   int plain64;  // the plain FP16-arithmetic hop on 64-site blocks (Ls <= 16)
   const CgState* cg;  // optional: blocks of columns with cg->mode != 0 do nothing
+  const unsigned* nbt;  // neighbour table (launch_neighbours); three-phase kernels
+  unsigned nblk;        // blocks per column and the division by their number (set by the launcher)
+  FastDiv dncol;
 };
 
 // Scalars of the FP64 CG on the device, one slot for the even and one for
@@ -424,6 +427,9 @@ void launch_prop_col_to_5d(const double2* src, double2* soa, const LatGeo& g, in
 void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, int ls, int eo, int col,
                            hipStream_t st);
 // l16 (optional): FP16 copy of the links, h16x2 (re, im) per element
+// Device half-site index of the neighbours of every site: nbt[(p * 8 + d) *
+// stride + h], p the parity slot of h (0 even, 1 odd), d as in neighbour_of.
+void launch_neighbours(unsigned* nbt, const LatGeo& g, hipStream_t st);
 void launch_pack_gauge(const double2* gauge, double2* l64, float2* l32, unsigned* l16, const LatGeo& g,
                        hipStream_t st);
 

@@ -191,6 +191,18 @@ void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, in
   hipLaunchKernelGGL(k_5d_to_prop_col, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, soa, dst, g, ls, eo, col);
 }
 
+__global__ void __launch_bounds__(kBlasBlock) k_neighbours(unsigned* __restrict__ nbt, LatGeo g)
+{
+  const int64_t h = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x;
+  const int pd = blockIdx.y;  // p * 8 + d
+  if (h < g.vh) nbt[pd * g.stride + h] = (unsigned)neighbour_of(g, h, pd < 8 ? 2 : 1, pd & 7);
+}
+void launch_neighbours(unsigned* nbt, const LatGeo& g, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_neighbours, dim3((unsigned)((g.vh + kBlasBlock - 1) / kBlasBlock), 16), dim3(kBlasBlock), 0, st,
+                     nbt, g);
+}
+
 // Gauge AoS [site][mu][3][3] complex128 -> per-output-parity 8-link layout
 // (dwf_common.h), FP64 and FP32 copies.  Backward links are stored already
 // adjointed: U_mu(x - mu)^+.

@@ -302,23 +302,29 @@ __device__ __forceinline__ void store_qs(typename SpinorIO<ST>::slot_t* __restri
 
 // HM: 0 FP32 arithmetic in the hop phase (8 neighbour spinors in flight per
 // thread, a register budget of 3 waves per SIMD); 1 FP16 arithmetic
-// (hop_term_h2) with 4 neighbour spinors in flight and 4 waves per SIMD.
-// Measured at 24^3x64 Ls12 over 4 columns (b = K H t): 1.177 ms and
-// 1.063 ms; FP16 arithmetic with 8 in flight needs 129 registers (3
-// waves per SIMD, 1.28 ms), or spills when held to 128.
-template <int HM>
+// (hop_term_h2) with 4 neighbour spinors in flight and 5 waves per SIMD (4
+// where the complex s-matrices of more than 16 rows take the LDS of a fifth).
+// The FP16 kernels are bound by VALU issue (70-76% busy in counters).  Site
+// places from the neighbour table, power-of-two scales, one v_max3 per pair,
+// first terms assigned instead of added to zeros and streamed inputs taken
+// without an unscaled copy leave 1001 of 1216 instructions in b = K H t, 833
+// of 999 in the plain hop and 1336 of 1658 in the hop with the dot product:
+// the operator 188 -> 163 us a column at 16^3x32 Ls12 with 4 columns and 166
+// -> 163 with 12, 24^3x64 Ls12 with 12 columns 1237 -> 1107 us.  A budget of
+// 6 waves spills in the s-matrix phase: 1115 against 1093 us there.
+template <int HM, int LSMAX, bool REAL>
 struct HopMode {
   static constexpr bool h2 = HM != 0;
   static constexpr int nb = HM ? 4 : 8;
-  static constexpr int wpe = HM ? 4 : 3;
+  static constexpr int wpe = HM ? (LSMAX > 16 && !REAL ? 4 : 5) : 3;
 };
 
 template <class ST, int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT, bool SMAT, int HM>
-__global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(HopMode<HM>::wpe)))
+__global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(HopMode<HM, LSMAX, REAL>::wpe)))
 k_hop_m5s(HopM5Args a)
 {
   typedef typename SpinorIO<ST>::slot_t slot_t;
-  constexpr bool H2 = HopMode<HM>::h2;
+  constexpr bool H2 = HopMode<HM, LSMAX, REAL>::h2;
   static_assert(!H2 || std::is_same<ST, Half16>::value, "FP16 arithmetic needs FP16 storage");
   // links of the block's sites: FP32 complex, or (H2) the FP16 forms
   // la = (re, -im), lb = (im, re) of hop_term_h2
@@ -336,14 +342,20 @@ k_hop_m5s(HopM5Args a)
   __shared__ h16x2 sla_own[LO][LS_], slb_own[LO][LS_];
   h16x2(*sla)[SB] = ALIAS ? (h16x2(*)[SB])pool : (h16x2(*)[SB])sla_own;
   h16x2(*slb)[SB] = ALIAS ? (h16x2(*)[SB])(pool + 72u * SB * 4u) : (h16x2(*)[SB])slb_own;
-  // block numbers are below 2^32: 32-bit divisions
-  const unsigned lbc = (unsigned)xcd_logical_block(blockIdx.x, (int64_t)gridDim.x);
+  const unsigned lbc = xcd_logical_block32(blockIdx.x, gridDim.x);
   const int ncol = a.cols.n;
-  const unsigned nblk = gridDim.x / (unsigned)ncol;
+  const unsigned nblk = a.nblk;  // blocks per column
   // column-fastest (the columns of a site block back to back: link reuse)
   // or site-fastest (one column's sites back to back: neighbour reuse)
-  const unsigned lb = a.site_major ? lbc % nblk : lbc / (unsigned)ncol;
-  const int ci = a.site_major ? (int)(lbc / nblk) : (int)(lbc - lb * (unsigned)ncol);
+  unsigned lb, cu;
+  if (a.site_major) {
+    cu = lbc / nblk;
+    lb = lbc - cu * nblk;
+  } else {
+    lb = fdiv(lbc, a.dncol);
+    cu = lbc - lb * (unsigned)ncol;
+  }
+  const int ci = (int)cu;
   if (a.cg && a.cg->mode[ci] != 0) return;  // frozen column (the whole block)
   const int64_t h0 = (int64_t)lb * SB;
   const int pslot = (a.eo_out == 2) ? 0 : 1;
@@ -380,12 +392,18 @@ k_hop_m5s(HopM5Args a)
   } else if constexpr (SMAT) {
     stage_km<LSMAX>(km, pick(a.mats, ci), a.ls);
   }
-  // neighbour indices once per site, shared by the Ls rows (thread (site,
-  // d) of the first 8 SB forms neighbour d of its site)
-  __shared__ unsigned nbs[8][SB];
+  // where neighbour d of each site starts in a field (row 0), formed once
+  // per site from the neighbour table and shared by the Ls rows; with FP16
+  // arithmetic and an s-matrix phase behind the links in the pool, which the
+  // hop results take over
+  typedef typename SpinorIO<ST>::At At;
+  static_assert(!ALIAS || kLinkBytes + 8u * SB * sizeof(At) <= (kLinkBytes > kHrBytes ? kLinkBytes : kHrBytes), "pool");
+  __shared__ At nbs_own[ALIAS ? 1 : 8][ALIAS ? 1 : SB];
+  At(*nbs)[SB] = ALIAS ? (At(*)[SB])(pool + kLinkBytes) : (At(*)[SB])nbs_own;
+  const unsigned* __restrict__ nbt = a.nbt + (int64_t)pslot * 8 * a.geo.stride + h0;
   for (int i = threadIdx.x; i < 8 * SB; i += blockDim.x) {
     const int st = i % SB, d = i / SB;
-    if (h0 + st < a.geo.vh) nbs[d][st] = (unsigned)neighbour_of(a.geo, h0 + st, a.eo_out, d);
+    if (h0 + st < a.geo.vh) nbs[d][st] = SpinorIO<ST>::at(a.ls, nbt[d * a.geo.stride + st]);
   }
   __syncthreads();
   const int ls = a.ls;
@@ -393,21 +411,20 @@ k_hop_m5s(HopM5Args a)
   const int64_t h = h0 + site;
   const bool active = h < a.geo.vh;
   const int64_t coff = (int64_t)pick(a.cols.rhs, ci) * a.cols.fstride;
-  cplx<float> acc[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) acc[k] = cmk<float>(0, 0);
+  cplx<float> acc[12];  // (set by active threads only)
   if (active && row < ls) {
-    unsigned nb[8];
-#pragma unroll
-    for (int d = 0; d < 8; ++d) nb[d] = nbs[d][site];
     const slot_t* __restrict__ in = (const slot_t*)a.in + coff;
     constexpr int SF = DAG ? 1 : -1;
     constexpr int SB_ = -SF;
+    if constexpr (!H2) {
+#pragma unroll
+      for (int k = 0; k < 12; ++k) acc[k] = cmk<float>(0, 0);
+    }
     // neighbour spinors are loaded in batches of NB directions before any
     // of them is used, so that each wave keeps several gathers in flight
-    constexpr int NB = std::is_same<ST, Half16>::value ? HopMode<HM>::nb : 4;
+    constexpr int NB = std::is_same<ST, Half16>::value ? HopMode<HM, LSMAX, REAL>::nb : 4;
     typename SpinorIO<ST>::Raw raw[NB];
-#define QDWF_LD(J, D) SpinorIO<ST>::load_raw(in, ls, row, nb[D], raw[J]);
+#define QDWF_LD(J, D) SpinorIO<ST>::load_raw(in, nbs[D][site], row, raw[J]);
 #define QDWF_CP(J, D, MU, SG)                                       \
   if constexpr (H2) {                                               \
     h16x2 la[9], lb[9], hp[12];                                     \
@@ -423,7 +440,7 @@ k_hop_m5s(HopM5Args a)
       hp[4 * j + 2] = __builtin_bit_cast(h16x2, raw[J].q[j].z);     \
       hp[4 * j + 3] = __builtin_bit_cast(h16x2, raw[J].q[j].w);     \
     }                                                               \
-    hop_term_h2<MU, SG>(la, lb, hp, raw[J].sc, acc);                \
+    hop_term_h2<MU, SG, (D) == 0>(la, lb, hp, raw[J].sc, acc);      \
   } else {                                                          \
     cplx<float> W[9];                                               \
     _Pragma("unroll") for (int e = 0; e < 9; ++e)                   \
@@ -483,32 +500,28 @@ k_hop_m5s(HopM5Args a)
       __syncthreads();
       if (active && row < ls) smat_row<SB, LSMAX, REAL>(hr, km, ls, site, row, v);
     }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) v[k] = cmk<float>(sc * acc[k].re, sc * acc[k].im);
   }
   double dot = 0.0, dotr = 0.0, dota = 0.0;
   if (active && row < ls) {
-    if (XPAY) {  // (the streamed inputs are read with non-temporal loads)
-      cplx<float> xv[12];
-      SpinorIO<ST>::load_stream((const slot_t*)a.x + coff, ls, row, h, xv);
+    if constexpr (!SMAT) {
 #pragma unroll
-      for (int k = 0; k < 12; ++k) v[k] = cmk<float>(v[k].re + a.beta * xv[k].re, v[k].im + a.beta * xv[k].im);
+      for (int k = 0; k < 12; ++k) v[k] = cmk<float>(sc * acc[k].re, sc * acc[k].im);
     }
+    if (XPAY)  // (the streamed inputs are read with non-temporal loads)
+      SpinorIO<ST>::fma_stream((const slot_t*)a.x + coff, ls, row, h, a.beta, v);
     store_qs<ST>((slot_t*)a.out + coff, ls, row, h, v);
     if (DOT) {
-      cplx<float> pv[12];
-      SpinorIO<ST>::load_stream((const slot_t*)a.dotp + coff, ls, row, h, pv);
-#pragma unroll
-      for (int k = 0; k < 12; ++k) dot += (double)pv[k].re * v[k].re + (double)pv[k].im * v[k].im;
+      dot = SpinorIO<ST>::dot_stream((const slot_t*)a.dotp + coff, ls, row, h, v);
       if (a.dotr) {
         cplx<float> rv[12];
         SpinorIO<float>::load_stream((const float4*)a.dotr + (int64_t)pick(a.cols.rhs, ci) * a.dotr_fstride, ls,
                                      row, h, rv);
 #pragma unroll
         for (int k = 0; k < 12; ++k) {
-          dotr += (double)rv[k].re * v[k].re + (double)rv[k].im * v[k].im;
-          dota += (double)v[k].re * v[k].re + (double)v[k].im * v[k].im;
+          dotr = fma((double)rv[k].re, (double)v[k].re, dotr);
+          dotr = fma((double)rv[k].im, (double)v[k].im, dotr);
+          dota = fma((double)v[k].re, (double)v[k].re, dota);
+          dota = fma((double)v[k].im, (double)v[k].im, dota);
         }
       }
     }
@@ -536,11 +549,21 @@ k_hop_m5s(HopM5Args a)
   }
 }
 
+template <int SB>
+static HopM5Args number_blocks(const HopM5Args& a)
+{
+  HopM5Args b = a;
+  b.nblk = (unsigned)((a.geo.vh + SB - 1) / SB);
+  b.dncol = make_fastdiv((unsigned)a.cols.n);
+  return b;
+}
+
 // plain hop: out = alpha H in + beta x (no s-matrix phase)
 template <class ST, int SB, int LSMAX, int H2>
-static void launch_hop_plain_ls(const HopM5Args& a, bool dag, hipStream_t st)
+static void launch_hop_plain_ls(const HopM5Args& a0, bool dag, hipStream_t st)
 {
-  const dim3 grid((unsigned)((a.geo.vh + SB - 1) / SB * a.cols.n));
+  const HopM5Args a = number_blocks<SB>(a0);
+  const dim3 grid(a.nblk * (unsigned)a.cols.n);
   const dim3 blk(SB * a.ls);
   const bool xpay = a.x != nullptr;
   if (!dag && !xpay) hipLaunchKernelGGL((k_hop_m5s<ST, SB, LSMAX, false, false, true, false, false, H2>), grid, blk, 0, st, a);
@@ -550,9 +573,10 @@ static void launch_hop_plain_ls(const HopM5Args& a, bool dag, hipStream_t st)
 }
 
 template <class ST, int SB, int LSMAX, int H2>
-static void launch_hop_m5s_ls(const HopM5Args& a, bool dag, hipStream_t st)
+static void launch_hop_m5s_ls(const HopM5Args& a0, bool dag, hipStream_t st)
 {
-  const dim3 grid((unsigned)((a.geo.vh + SB - 1) / SB * a.cols.n));
+  const HopM5Args a = number_blocks<SB>(a0);
+  const dim3 grid(a.nblk * (unsigned)a.cols.n);
   const dim3 blk(SB * a.ls);
   const bool xpay = a.x != nullptr;
 #define QDWF_L(D, X, R, DT) hipLaunchKernelGGL((k_hop_m5s<ST, SB, LSMAX, D, X, R, DT, true, H2>), grid, blk, 0, st, a)
