@@ -252,7 +252,7 @@ struct qlat_dwf_inverter {
   bool fused32 = true;  // FP32 hop + s-matrix fusion (QLAT_DWF_FUSED=0 disables)
   bool three_phase32 = true;   // FP32 solver on the three-phase kernels (QLAT_DWF_THREE_PHASE=0: fused
                                // FP32 kernels, single s-matrix pass per hop)
-  int tp_sb = 32;              // sites per block of the three-phase kernels (QLAT_DWF_TP_SB)
+  int tp_sb = 0;               // sites per block of the three-phase kernels (QLAT_DWF_TP_SB; 0: default_sb)
   int step_sb = 32;            // sites per block of the three-phase CG step (QLAT_DWF_STEP_SB)
   bool x_defer = true;         // x updated every other CG step, two directions at once (QLAT_DWF_XDEFER)
   int site_major = 0;          // three-phase hop block order (QLAT_DWF_SITE_MAJOR)
@@ -1144,6 +1144,23 @@ void deflate_dev(Inv& I, double2* out, const double2* in, int eo)
   check_launch();
 }
 
+// Sites per block of the three-phase kernels where the autotuner does not
+// choose them (single columns, fixed tiles): 16, the smallest block of whole
+// waves, and 32 where Ls is no multiple of 4.  Solves of one column, 16
+// against 32 sites: FP32 24^3x64 Ls12 0.83 against 0.93 s, 16^3x32 Ls12 95
+// against 108 ms and Ls16 128 against 144 ms, FP16 storage 16^3x32 Ls12 68
+// against 74 ms, 8^3x16 Ls12 11.4 against 12.2 ms.  From 16^3x32 up Ls 8
+// keeps 32 (56.7 against 58.0 ms: blocks of two waves otherwise) and Ls 24
+// takes 8 (216 against 223 ms: three blocks of LDS more per CU).
+int default_sb(const Inv& I)
+{
+  if (I.tp_sb) return I.tp_sb;
+  const bool large = I.geo.vh >= 1 << 16;
+  if (large && I.ls == 8) return 32;
+  if (large && I.ls == 24) return 8;
+  return I.ls % 4 ? 32 : 16;
+}
+
 struct ThreePhase {
   Inv& I;
   int storage;
@@ -1163,7 +1180,7 @@ struct ThreePhase {
   // buffer of the eager loop
   double* red_out = nullptr;
   ThreePhase(Inv& inv, int ncol, int storage_, int sb_ = 0)
-      : I(inv), storage(storage_), sb(sb_ ? sb_ : inv.tp_sb), red_out(inv.red)
+      : I(inv), storage(storage_), sb(sb_ ? sb_ : default_sb(inv)), red_out(inv.red)
   {
     if (!qdwf::three_phase_ok(I.ls, sb))
       for (int alt : {16, 32, 8})
@@ -1773,7 +1790,7 @@ TileChoice autotune_tile(Inv& I, int storage, int ncol)
 // (with QLAT_DWF_TP_SB) when set, else the autotuner's choice.
 TileChoice tile_for(Inv& I, int storage, int ncol)
 {
-  if (I.rhs_tile > 0) return TileChoice{I.rhs_tile, I.tp_sb};
+  if (I.rhs_tile > 0) return TileChoice{I.rhs_tile, default_sb(I)};
   return autotune_tile(I, storage, ncol);
 }
 
@@ -2157,7 +2174,7 @@ long solve_columns(Inv& I, int n, Inv* const* colinv, Load&& load, Store&& store
   for (int j = 0; j < n; ++j) several = several || colinv[j] != &I;
   const bool three = use_three_phase(I) || (several && qdwf::three_phase_ls_ok(I.ls));
   const int storage = storage_of(I);
-  TileChoice tc{I.rhs_tile > 0 ? I.rhs_tile : 12, I.tp_sb};
+  TileChoice tc{I.rhs_tile > 0 ? I.rhs_tile : 12, default_sb(I)};
   if (three) tc = tile_for(I, storage, n);
   tc.width = std::max(1, std::min(tc.width, qdwf::kMaxRhs));
   I.stats.rhs_tile = tc.width;
