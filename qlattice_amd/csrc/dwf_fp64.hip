@@ -274,15 +274,14 @@ void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st)
 // requested as soon as the current one has been projected to its half
 // spinor, so that a wave always has 12 loads in flight while it multiplies
 // (acc, the loads and the half spinor are 144 of 168 registers: 3 waves per
-// SIMD).
-template <bool DAG, class Load, class Link>
-__device__ __forceinline__ void hop_acc_d(Load&& load, Link&& link, cplx<double> acc[12])
+// SIMD).  raw holds neighbour 0 already; last(raw) may request
+// something else into it behind the last direction's products.
+template <bool DAG, class Load, class Link, class Last>
+__device__ __forceinline__ void hop_acc_d(Load&& load, Link&& link, Last&& last, double2 raw[12], cplx<double> acc[12])
 {
   constexpr int SF = DAG ? 1 : -1, SG = -SF;
 #pragma unroll
   for (int k = 0; k < 12; ++k) acc[k] = cmk<double>(0, 0);
-  double2 raw[12];
-  load(0, raw);
 #define QDWF_D(D, MU, SGN, NEXT)                                                                        \
   {                                                                                                     \
     cplx<double> w0[3], w1[3];                                                                          \
@@ -290,6 +289,7 @@ __device__ __forceinline__ void hop_acc_d(Load&& load, Link&& link, cplx<double>
         cmk<double>(raw[c].x, raw[c].y), cmk<double>(raw[3 + c].x, raw[3 + c].y),                       \
         cmk<double>(raw[6 + c].x, raw[6 + c].y), cmk<double>(raw[9 + c].x, raw[9 + c].y), w0[c], w1[c]); \
     if (NEXT >= 0) load(NEXT, raw);                                                                     \
+    else last(raw);                                                                                     \
     _Pragma("unroll") for (int r = 0; r < 3; ++r)                                                       \
     {                                                                                                   \
       const cplx<double> u0 = link((D) * 9 + r * 3), u1 = link((D) * 9 + r * 3 + 1),                    \
@@ -337,7 +337,9 @@ __device__ __forceinline__ void stage_links_d(double2 (*sl)[SB], int (*nbs)[SB],
 // the sites in flight on its 32 CUs are larger than that, so a spinor is
 // fetched about three times per launch (24^3x64 Ls12, 0.81 ms).  Before the
 // links' loads were batched and the next spinor requested early: 0.88 ms, at
-// 16^3x32 Ls8 91 us (now 64), at 8^3x16 Ls12 28 us (now 7).
+// 16^3x32 Ls8 91 us (now 64), at 8^3x16 Ls12 28 us (now 7).  x is requested
+// behind the last direction's products: inside Mpc^+ Mpc 98 against 109 us at
+// 16^3x32 Ls8, 10.2 against 11.8 us at 8^3x16 Ls8.
 template <int SB, int NW, bool DAG, bool XPAY, bool NT>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB == 64 ? 2 : 3))) k_hop_d(HopArgs<double> a)
 {
@@ -356,29 +358,35 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB
     // the links stay in LDS: read anew for every row (hoisted out of the
     // loop they would take 288 registers)
     asm volatile("" ::: "memory");
-    cplx<double> acc[12];
-    hop_acc_d<DAG>(
-        [&](int d, double2 raw[12]) {
-          const double2* __restrict__ p = in + sidx<12>(a.ls, s, 0, nbs[d][site]);
+    auto load = [&](int d, double2 raw[12]) {
+      const double2* __restrict__ p = in + sidx<12>(a.ls, s, 0, nbs[d][site]);
 #pragma unroll
-          for (int k = 0; k < 12; ++k) raw[k] = p[k * 64];
-        },
+      for (int k = 0; k < 12; ++k) raw[k] = p[k * 64];
+    };
+    cplx<double> acc[12];
+    double2 raw[12];
+    load(0, raw);
+    hop_acc_d<DAG>(
+        load,
         [&](int i) {
           const double2 u = sl[i][site];
           return cmk<double>(u.x, u.y);
         },
-        acc);
+        [&](double2 xv[12]) {
+          if (!XPAY) return;
+          const double2* __restrict__ x = (const double2*)a.x + sidx<12>(a.ls, s, 0, h);
+#pragma unroll
+          for (int k = 0; k < 12; ++k) xv[k] = load_in<NT>(&x[k * 64]);
+          __builtin_amdgcn_sched_barrier(0);  // (not to be moved behind the products)
+        },
+        raw, acc);
     cplx<double> v[12];
 #pragma unroll
     for (int k = 0; k < 12; ++k) v[k] = cmk<double>(sc * acc[k].re, sc * acc[k].im);
     if (XPAY) {
-      const double2* __restrict__ x = (const double2*)a.x + sidx<12>(a.ls, s, 0, h);
       const cplx<double> b = a.beta[s];
 #pragma unroll
-      for (int k = 0; k < 12; ++k) {
-        const double2 xv = load_in<NT>(&x[k * 64]);
-        v[k] = cfma(v[k], b, cmk<double>(xv.x, xv.y));
-      }
+      for (int k = 0; k < 12; ++k) v[k] = cfma(v[k], b, cmk<double>(raw[k].x, raw[k].y));
     }
     SpinorIO<double>::store_stream((double2*)a.out, a.ls, s, h, v);
   }
@@ -417,7 +425,8 @@ void launch_hop_d(const HopArgs<double>& a, bool dag, hipStream_t st)
 // after the other (half the LDS), and the waves take the (component, 16
 // sites) pairs of the s-matrix product in turn.  Bound like k_hop_d: 0.93 ms
 // at 24^3x64 Ls12; 80 us at 16^3x32 Ls8 (97 with the product row by row from
-// LDS on the vector units), 11 us at 8^3x16 Ls8.
+// LDS on the vector units), 11 us at 8^3x16 Ls8.  With x and the dot product
+// 117 and 14 us, 108 and 12 us with dotp requested before the s-matrix product.
 template <int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT, bool NT>
 __global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(3))) k_hop_m5d(HopM5dArgs a)
 {
@@ -435,17 +444,20 @@ __global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu
   const int site = threadIdx.x % SB, row = threadIdx.x / SB;
   cplx<double> acc[12];
   if (h0 + site < a.geo.vh && row < ls) {
-    hop_acc_d<DAG>(
-        [&](int d, double2 raw[12]) {
-          const double2* __restrict__ p = a.in + sidx<12>(ls, row, 0, nbs[d][site]);
+    auto load = [&](int d, double2 raw[12]) {
+      const double2* __restrict__ p = a.in + sidx<12>(ls, row, 0, nbs[d][site]);
 #pragma unroll
-          for (int k = 0; k < 12; ++k) raw[k] = p[k * 64];
-        },
+      for (int k = 0; k < 12; ++k) raw[k] = p[k * 64];
+    };
+    double2 raw[12];
+    load(0, raw);
+    hop_acc_d<DAG>(
+        load,
         [&](int i) {
           const double2 u = buf[i][site];
           return cmk<double>(u.x, u.y);
         },
-        acc);
+        [](double2*) {}, raw, acc);
   } else {  // (rows beyond ls are operands of the products)
 #pragma unroll
     for (int k = 0; k < 12; ++k) acc[k] = cmk<double>(0, 0);
@@ -472,14 +484,17 @@ __global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu
       mf4d dr[Mx::MT], di[Mx::MT];
 #pragma unroll
       for (int mt = 0; mt < Mx::MT; ++mt) dr[mt] = di[mt] = (mf4d){0.0, 0.0, 0.0, 0.0};
-      double2 xv[Mx::MT][4];
-      if (XPAY) {
+      constexpr bool EARLY = DOT && Mx::MT == 1;  // (two row tiles have no registers for it)
+      double2 xv[Mx::MT][4], pv[Mx::MT][4];
+      if (XPAY || EARLY) {
 #pragma unroll
         for (int mt = 0; mt < Mx::MT; ++mt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int s = mt * 16 + lq + 4 * i;
-            if (act && s < ls) xv[mt][i] = load_in<NT>(&a.x[sidx<12>(ls, s, chi * 6 + k, h)]);
+            const unsigned o = sidx<12>(ls, s, chi * 6 + k, h);
+            if (XPAY && act && s < ls) xv[mt][i] = load_in<NT>(&a.x[o]);
+            if (EARLY && act && s < ls) pv[mt][i] = load_in<NT>(&a.dotp[o]);
           }
       }
 #pragma unroll
@@ -499,7 +514,7 @@ __global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu
           }
           store_nt(&a.out[o], v);
           if (DOT) {
-            const double2 p = load_in<NT>(&a.dotp[o]);
+            const double2 p = EARLY ? pv[mt][i] : load_in<NT>(&a.dotp[o]);
             dot += p.x * v.x + p.y * v.y;
           }
         }
