@@ -427,6 +427,13 @@ void launch_prop_col_to_5d(const double2* src, double2* soa, const LatGeo& g, in
 void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, int ls, int eo, int col,
                            hipStream_t st);
 // l16 (optional): FP16 copy of the links, h16x2 (re, im) per element
+// Copies between host and device memory on a stream, complete for the host
+// array on return (the device side of copy_to_device is in stream order).
+// The staging ring lives while a retain is held.
+void copy_ring_retain();
+void copy_ring_release();
+hipError_t copy_to_device(int device, hipStream_t st, void* dev, const void* host, size_t bytes, size_t ring_min = 0);
+hipError_t copy_to_host(int device, hipStream_t st, void* host, const void* dev, size_t bytes);
 // Device half-site index of the neighbours of every site: nbt[(p * 8 + d) *
 // stride + h], p the parity slot of h (0 even, 1 odd), d as in neighbour_of.
 void launch_neighbours(unsigned* nbt, const LatGeo& g, hipStream_t st);
