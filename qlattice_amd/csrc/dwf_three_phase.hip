@@ -300,47 +300,57 @@ __device__ __forceinline__ void store_qs(typename SpinorIO<ST>::slot_t* __restri
   else SpinorIO<ST>::store_stream(f, ls, s, h, v);
 }
 
-// HM: 0 FP32 arithmetic in the hop phase (8 neighbour spinors in flight per
-// thread, a register budget of 3 waves per SIMD); 1 FP16 arithmetic
-// (hop_term_h2) with 4 neighbour spinors in flight and 5 waves per SIMD (4
-// where the complex s-matrices of more than 16 rows take the LDS of a fifth).
+// HM: 0 FP32 arithmetic in the hop phase, 2 neighbour spinors of a thread in
+// flight; 1 FP16 arithmetic (hop_term_h2), 3 in flight; 5 waves per SIMD (fewer
+// where LDS has no room for them).
+// FP32: bound by what it fetches, 0.41 ms for b = K H t at 24^3x64 Ls12.
+// Against batches of 4 spinors with 3 waves Mpc^+ Mpc takes 1924 instead of
+// 1947 us there, 176 instead of 184 at 16^3x32 Ls8, 543 instead of 579 at Ls24;
+// batches with 4 waves spill.
 // The FP16 kernels are bound by VALU issue (70-76% busy in counters).  Site
 // places from the neighbour table, power-of-two scales, one v_max3 per pair,
 // first terms assigned instead of added to zeros and streamed inputs taken
 // without an unscaled copy leave 1001 of 1216 instructions in b = K H t, 833
 // of 999 in the plain hop and 1336 of 1658 in the hop with the dot product:
-// the operator 188 -> 163 us a column at 16^3x32 Ls12 with 4 columns and 166
-// -> 163 with 12, 24^3x64 Ls12 with 12 columns 1237 -> 1107 us.  A budget of
-// 6 waves spills in the s-matrix phase: 1115 against 1093 us there.
-template <int HM, int LSMAX, bool REAL>
+// the operator 188 -> 155 us a column at 16^3x32 Ls12 with 4 columns, 24^3x64
+// Ls12 with 12 columns 1237 -> 1105 us; rings of 3 instead of batches of 4
+// spinors leave 152 and 1086 us.  A budget of 6 waves spills in the s-matrix
+// phase: 1115 against 1093 us.
+template <int HM, int SB, int LSMAX, bool REAL, bool SMAT>
 struct HopMode {
   static constexpr bool h2 = HM != 0;
-  static constexpr int nb = HM ? 4 : 8;
-  static constexpr int wpe = HM ? (LSMAX > 16 && !REAL ? 4 : 5) : 3;
+  static constexpr int nb = HM ? 3 : 2;
+  // blocks of a CU by LDS: links, or the hop results in their place, and the
+  // s-matrices (real parts alone on the matrix-core paths)
+  static constexpr int link = 576 * SB, hr = 96 * LSMAX * SB;
+  static constexpr int km = SMAT ? 2 * LSMAX * LSMAX * (REAL && SB <= 16 ? 4 : 8) : 64 * SB;
+  static constexpr int lds = (SMAT && hr > link ? hr : link) + km + 256;
+  static constexpr int waves = (SB * LSMAX + 63) / 64 * (160 * 1024 / lds) / 4;
+  static constexpr int wpe = waves > 5 ? 5 : waves > 1 ? waves : 1;
 };
 
 template <class ST, int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT, bool SMAT, int HM>
-__global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(HopMode<HM, LSMAX, REAL>::wpe)))
+__global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(HopMode<HM, SB, LSMAX, REAL, SMAT>::wpe)))
 k_hop_m5s(HopM5Args a)
 {
   typedef typename SpinorIO<ST>::slot_t slot_t;
-  constexpr bool H2 = HopMode<HM, LSMAX, REAL>::h2;
+  constexpr bool H2 = HopMode<HM, SB, LSMAX, REAL, SMAT>::h2;
   static_assert(!H2 || std::is_same<ST, Half16>::value, "FP16 arithmetic needs FP16 storage");
   // links of the block's sites: FP32 complex, or (H2) the FP16 forms
   // la = (re, -im), lb = (im, re) of hop_term_h2
-  __shared__ float2 sl[H2 ? 1 : 72][H2 ? 1 : SB];
-  // With FP16 arithmetic and an s-matrix phase the links and the hop
-  // results (hr below) share one LDS area; the hop phase ends at a barrier
-  // before the results go in.  With the real matrices' real parts staged
-  // alone (kmr below) a 16-site block at Ls 12 takes 20 KB instead of 30 KB:
-  // 8 blocks per CU instead of 5
-  constexpr bool ALIAS = H2 && SMAT;
+  // With an s-matrix phase the links and the hop results (hr below) share
+  // one LDS area; the hop phase ends at a barrier before the results go in.
+  // With the real matrices' real parts staged alone (kmr below) a 16-site
+  // block at Ls 12 takes 20 KB instead of 30 KB: 8 blocks per CU instead of 5
+  constexpr bool ALIAS = SMAT;
   constexpr unsigned kLinkBytes = 2u * 72u * SB * 4u;
   constexpr unsigned kHrBytes = (unsigned)LSMAX * 6u * SB * 16u;
   __shared__ __attribute__((aligned(16))) unsigned char pool[ALIAS ? (kLinkBytes > kHrBytes ? kLinkBytes : kHrBytes) : 16];
   constexpr int LO = H2 && !ALIAS ? 72 : 1, LS_ = H2 && !ALIAS ? SB : 1;
   __shared__ h16x2 sla_own[LO][LS_], slb_own[LO][LS_];
   h16x2(*sla)[SB] = ALIAS ? (h16x2(*)[SB])pool : (h16x2(*)[SB])sla_own;
+  __shared__ float2 sl_own[!H2 && !ALIAS ? 72 : 1][!H2 && !ALIAS ? SB : 1];
+  float2(*sl)[SB] = ALIAS ? (float2(*)[SB])pool : (float2(*)[SB])sl_own;
   h16x2(*slb)[SB] = ALIAS ? (h16x2(*)[SB])(pool + 72u * SB * 4u) : (h16x2(*)[SB])slb_own;
   const unsigned lbc = xcd_logical_block32(blockIdx.x, gridDim.x);
   const int ncol = a.cols.n;
@@ -393,9 +403,9 @@ k_hop_m5s(HopM5Args a)
     stage_km<LSMAX>(km, pick(a.mats, ci), a.ls);
   }
   // where neighbour d of each site starts in a field (row 0), formed once
-  // per site from the neighbour table and shared by the Ls rows; with FP16
-  // arithmetic and an s-matrix phase behind the links in the pool, which the
-  // hop results take over
+  // per site from the neighbour table and shared by the Ls rows; with an
+  // s-matrix phase behind the links in the pool, which the hop results take
+  // over
   typedef typename SpinorIO<ST>::At At;
   static_assert(!ALIAS || kLinkBytes + 8u * SB * sizeof(At) <= (kLinkBytes > kHrBytes ? kLinkBytes : kHrBytes), "pool");
   __shared__ At nbs_own[ALIAS ? 1 : 8][ALIAS ? 1 : SB];
@@ -420,9 +430,9 @@ k_hop_m5s(HopM5Args a)
 #pragma unroll
       for (int k = 0; k < 12; ++k) acc[k] = cmk<float>(0, 0);
     }
-    // neighbour spinors are loaded in batches of NB directions before any
-    // of them is used, so that each wave keeps several gathers in flight
-    constexpr int NB = std::is_same<ST, Half16>::value ? HopMode<HM, LSMAX, REAL>::nb : 4;
+    // NB neighbour spinors of a thread in a ring: a direction's is requested
+    // NB - 1 directions before it is used
+    constexpr int NB = HopMode<HM, SB, LSMAX, REAL, SMAT>::nb;
     typename SpinorIO<ST>::Raw raw[NB];
 #define QDWF_LD(J, D) SpinorIO<ST>::load_raw(in, nbs[D][site], row, raw[J]);
 #define QDWF_CP(J, D, MU, SG)                                       \
@@ -452,17 +462,17 @@ k_hop_m5s(HopM5Args a)
     SpinorIO<ST>::decode(raw[J], psi);                              \
     hop_term<MU, SG>(W, psi, acc);                                  \
   }
-    if constexpr (NB == 8) {
-      QDWF_LD(0, 0) QDWF_LD(1, 1) QDWF_LD(2, 2) QDWF_LD(3, 3)
-      QDWF_LD(4, 4) QDWF_LD(5, 5) QDWF_LD(6, 6) QDWF_LD(7 % NB, 7)
-      QDWF_CP(0, 0, 0, SF) QDWF_CP(1, 1, 1, SF) QDWF_CP(2, 2, 2, SF) QDWF_CP(3, 3, 3, SF)
-      QDWF_CP(4 % NB, 4, 0, SB_) QDWF_CP(5 % NB, 5, 1, SB_) QDWF_CP(6 % NB, 6, 2, SB_) QDWF_CP(7 % NB, 7, 3, SB_)
-    } else {
-      QDWF_LD(0, 0) QDWF_LD(1, 1) QDWF_LD(2, 2) QDWF_LD(3, 3)
-      QDWF_CP(0, 0, 0, SF) QDWF_CP(1, 1, 1, SF) QDWF_CP(2, 2, 2, SF) QDWF_CP(3, 3, 3, SF)
-      QDWF_LD(0, 4) QDWF_LD(1, 5) QDWF_LD(2, 6) QDWF_LD(3, 7)
-      QDWF_CP(0, 4, 0, SB_) QDWF_CP(1, 5, 1, SB_) QDWF_CP(2, 6, 2, SB_) QDWF_CP(3, 7, 3, SB_)
-    }
+#define QDWF_D(D, MU, SG)                                       \
+  if constexpr ((D) + NB - 1 < 8) {                             \
+    QDWF_LD(((D) + NB - 1) % NB, ((D) + NB - 1) % 8)            \
+  }                                                             \
+  QDWF_CP((D) % NB, D, MU, SG)
+    static_assert(NB == 2 || NB == 3, "the loads requested before the first direction");
+    QDWF_LD(0, 0)
+    if constexpr (NB > 2) { QDWF_LD(1, 1) }
+    QDWF_D(0, 0, SF) QDWF_D(1, 1, SF) QDWF_D(2, 2, SF) QDWF_D(3, 3, SF)
+    QDWF_D(4, 0, SB_) QDWF_D(5, 1, SB_) QDWF_D(6, 2, SB_) QDWF_D(7, 3, SB_)
+#undef QDWF_D
 #undef QDWF_LD
 #undef QDWF_CP
   }
