@@ -75,7 +75,7 @@ struct MemError : std::runtime_error {
   } while (0)
 
 // ------------------------------------------------------------ s-matrices
-enum MatId { MAT_MEE, MAT_MEE_DAG, MAT_MEE_INV, MAT_MEE_INVDAG, MAT_P, MAT_P_DAG, MAT_K, MAT_K_DAG, MAT_NEGC, MAT_COUNT };
+enum MatId { MAT_MEE, MAT_MEE_DAG, MAT_MEE_INV, MAT_MEE_INVDAG, MAT_P, MAT_P_DAG, MAT_K, MAT_K_DAG, MAT_COUNT };
 
 typedef std::vector<cd> Mat;  // ls*ls row-major
 
@@ -273,7 +273,7 @@ struct qlat_dwf_inverter {
   int plain64 = 1;  // plain FP16 hop on 64-site blocks (QLAT_DWF_PLAIN64)
   cplx<double>* mat64 = nullptr;  // [MAT_COUNT][2][ls][ls]
   cplx<float>* mat32 = nullptr;
-  cplx<double>* beta64 = nullptr;  // [2][ls]: ones, c~
+  cplx<double>* beta64 = nullptr;  // [3][ls]: ones, c~, -c
   cplx<float>* beta32 = nullptr;
   double2* w64[W_COUNT64] = {};
   float4* w32[W_COUNT32] = {};
@@ -522,10 +522,11 @@ void m5(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, i
 template <class T>
 void hop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, int eo_out, bool dag,
          T alpha = 1, const typename Prec<T>::slot* x = nullptr, int beta = 0, const qdwf::RhsSet* cols = nullptr,
-         const qdwf::CgState64* cg = nullptr)
+         const qdwf::CgState64* cg = nullptr, const cplx<T>* gamma = nullptr)
 {
   qdwf::HopArgs<T> a;
   a.cg = cg;
+  a.gamma = gamma;
   a.cols = cols ? *cols : one_col();
   a.geo = I.geo;
   a.ls = I.ls;
@@ -767,6 +768,15 @@ double dev_norm2(Inv& I, const double2* a)
   sync(I);
   return I.red_map[0];
 }
+// |a|^2 + |b|^2
+double dev_norm2_sum(Inv& I, const double2* a, const double2* b)
+{
+  qdwf::launch_norm2<double2>(a, n64(I), I.part, I.red_map_dev, I.stream);
+  qdwf::launch_norm2<double2>(b, n64(I), I.part, I.red_map_dev + 1, I.stream);
+  check_launch();
+  sync(I);
+  return I.red_map[0] + I.red_map[1];
+}
 template <class S>
 cd dev_dot(Inv& I, const S* a, const S* b, int64_t n)
 {
@@ -792,27 +802,27 @@ void zero32(Inv& I, float4* dst) { QDWF_HIP(hipMemsetAsync(dst, 0, field32_bytes
 
 // --------------------------------------------------- full-lattice ops
 // multiply_d_minus (dslash.cpp:448-480): D_- psi = psi + D_W(-M5)(-c psi)
-//   = diag(c~) psi + H (-c psi), c~ = 1 - c (4 - M5)
+//   = diag(c~) psi + H (-c psi), c~ = 1 - c (4 - M5); c depends on s only, so
+// it is a factor of the hop's rows
 void op_d_minus(Inv& I, double2* out_e, double2* out_o, const double2* in_e, const double2* in_o)
 {
-  double2* t1 = W(I, W_OP_T1);
-  double2* t2 = W(I, W_OP_T2);
-  m5<double>(I, t1, in_o, MAT_NEGC);
-  m5<double>(I, t2, in_e, MAT_NEGC);
-  hop<double>(I, out_e, t1, 2, false, 1.0, in_e, 1);
-  hop<double>(I, out_o, t2, 1, false, 1.0, in_o, 1);
+  const cplx<double>* negc = Prec<double>::beta(I, 2);
+  hop<double>(I, out_e, in_o, 2, false, 1.0, in_e, 1, nullptr, nullptr, negc);
+  hop<double>(I, out_o, in_e, 1, false, 1.0, in_o, 1, nullptr, nullptr, negc);
 }
 
 // multiply_m (dslash.cpp:1062-1080): out_p = M_ee in_p + H P in_{3-p}
-void op_m_full(Inv& I, double2* out_e, double2* out_o, const double2* in_e, const double2* in_o)
+// (- sub_p)
+void op_m_full(Inv& I, double2* out_e, double2* out_o, const double2* in_e, const double2* in_o,
+               const double2* sub_e = nullptr, const double2* sub_o = nullptr)
 {
   double2* t1 = W(I, W_OP_T1);
   double2* t2 = W(I, W_OP_T2);
   m5<double>(I, t1, in_o, MAT_P);
-  m5<double>(I, t2, in_e, MAT_MEE);
+  m5<double>(I, t2, in_e, MAT_MEE, 1.0, sub_e, -1.0);
   hop<double>(I, out_e, t1, 2, false, 1.0, t2, 0);
   m5<double>(I, t1, in_e, MAT_P);
-  m5<double>(I, t2, in_o, MAT_MEE);
+  m5<double>(I, t2, in_o, MAT_MEE, 1.0, sub_o, -1.0);
   hop<double>(I, out_o, t1, 1, false, 1.0, t2, 0);
 }
 
@@ -887,6 +897,21 @@ long cg_fp64(Inv& I, double2* x, const double2* b, double stop_rsd, long max_num
   return max_num_iter + 1;
 }
 
+// |b - A x|^2 in FP64 for the operator of J, with r = scale (b - A x) in the
+// solver's storage (r may be null)
+double fp64_residual(Inv& I, Inv& J, const double2* b, const double2* x, void* r = nullptr, bool half = false,
+                     double scale = 1.0)
+{
+  double2* ax = W(I, W_CG_AP);
+  op_hermop<double>(J, ax, x, 1);
+  I.stats.hermop_fp64 += 1;
+  const int np = qdwf::launch_residual_d(b, ax, r, half, I.geo, I.ls, scale, I.part, I.stream);
+  qdwf::launch_reduce_rows(I.part, np, 1, I.red_map_dev, I.stream);
+  check_launch();
+  sync(I);
+  return I.red_map[0];
+}
+
 // Mixed-precision CG on A x = b (odd half fields) from the x64 it is given:
 // the Krylov recurrence runs in FP32; whenever the iterated residual has
 // dropped by `delta` since the last replacement (and at convergence) the
@@ -895,31 +920,20 @@ long cg_fp64(Inv& I, double2* x, const double2* b, double stop_rsd, long max_num
 // Returns iterations; stops when |b - A x| <= stop_rsd |b| in FP64.
 long cg_mixed(Inv& I, double2* x64, const double2* b64, double stop_rsd, long max_total_iter, double* true_rel)
 {
-  double2* r64 = W(I, W_CG_R);
-  double2* ax64 = W(I, W_CG_AP);
   float4* r = V(I, V_R);
   float4* p = V(I, V_P);
   float4* ap = V(I, V_AP);
   float4* x = V(I, V_X);
   float4* t = V(I, V_T);
-  const int64_t n = n32(I), nd = n64(I);
+  const int64_t n = n32(I);
   const double b2 = dev_norm2(I, b64);
   const double target = stop_rsd * stop_rsd * b2;
-  auto true_residual = [&]() {
-    op_hermop<double>(I, ax64, x64, 1);
-    I.stats.hermop_fp64 += 1;
-    copy64(I, r64, b64);
-    qdwf::launch_axpy<double2>(-1.0, ax64, r64, nd, I.stream);
-    check_launch();
-    return dev_norm2(I, r64);
-  };
+  auto true_residual = [&]() { return fp64_residual(I, I, b64, x64, r); };
   double rr = true_residual();
   if (rr <= target) {
     *true_rel = std::sqrt(rr / b2);
     return 0;
   }
-  qdwf::launch_d2f(r64, r, I.ls, I.geo.stride, I.stream);
-  check_launch();
   QDWF_HIP(hipMemcpyAsync(p, r, field32_bytes(I), hipMemcpyDeviceToDevice, I.stream));
   zero32(I, x);
   m5<float>(I, t, p, MAT_K);
@@ -948,8 +962,6 @@ long cg_mixed(Inv& I, double2* x64, const double2* b64, double stop_rsd, long ma
         *true_rel = std::sqrt(rr_true / b2);
         return iter;
       }
-      qdwf::launch_d2f(r64, r, I.ls, I.geo.stride, I.stream);
-      check_launch();
       rr_new = rr_true;
       maxrr = rr_true;
       cg_step(I, nullptr, p, r, t, 0.0, rr_new / rr);
@@ -976,7 +988,7 @@ void deflate_dev(Inv& I, double2* out, const double2* in, int eo);
 
 long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
 {
-  const int64_t fs = n32(I), nd = n64(I);
+  const int64_t fs = n32(I);
   float4* R = MV(I, M_R, ncol);
   float4* P = MV(I, M_P, ncol);
   float4* AP = MV(I, M_AP, ncol);
@@ -985,19 +997,10 @@ long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
   float4* B = MV(I, M_B, ncol);
   float4* Y = MV(I, M_Y, ncol);
   float4* A = I.fused32 ? B : MV(I, M_A, ncol);  // only the unfused path needs A
-  double2* r64 = W(I, W_CG_R);
-  double2* ax64 = W(I, W_CG_AP);
   std::vector<double> b2(ncol), target(ncol), rr(ncol), maxrr(ncol);
   std::vector<long> iters(ncol, 0);
   std::vector<int> active;
-  auto true_residual = [&](int c) {
-    op_hermop<double>(I, ax64, C64(I, c, 1), 1);
-    I.stats.hermop_fp64 += 1;
-    copy64(I, r64, C64(I, c, 0));
-    qdwf::launch_axpy<double2>(-1.0, ax64, r64, nd, I.stream);
-    check_launch();
-    return dev_norm2(I, r64);
-  };
+  auto true_residual = [&](int c) { return fp64_residual(I, I, C64(I, c, 0), C64(I, c, 1), R + c * fs); };
   for (int c = 0; c < ncol; ++c) {
     b2[c] = dev_norm2(I, C64(I, c, 0));
     target[c] = stop_rsd * stop_rsd * b2[c];
@@ -1006,8 +1009,6 @@ long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
       // deflated initial guess (dslash.h:496-500) in the FP64 x, r = b - A x
       deflate_dev(I, C64(I, c, 1), C64(I, c, 0), 1);
       rr[c] = maxrr[c] = true_residual(c);
-      qdwf::launch_d2f(r64, R + c * fs, I.ls, I.geo.stride, I.stream);
-      check_launch();
       if (rr[c] <= target[c]) {
         const double rel = std::sqrt(rr[c] / b2[c]);
         if (rel > I.stats.true_residual) I.stats.true_residual = rel;
@@ -1075,8 +1076,6 @@ long cg_mixed_multi(Inv& I, int ncol, double stop_rsd, long cap)
           if (rel > I.stats.true_residual) I.stats.true_residual = rel;
           continue;  // column retired
         }
-        qdwf::launch_d2f(r64, R + c * fs, I.ls, I.geo.stride, I.stream);
-        check_launch();
         rr_new[i] = rr_true;
         maxrr[c] = rr_true;
         step_alpha[i] = 0.0;
@@ -1480,22 +1479,14 @@ long cg_mixed_multi_s(Inv& I, int ncol, double2* const* b64, double2* const* x64
   ThreePhase tp(I, ncol, storage, sb);
   if (colinv)
     for (int c = 0; c < ncol; ++c) tp.colinv[c] = colinv[c];
-  const int64_t nd = n64(I);
-  double2* r64 = W(I, W_CG_R);
-  double2* ax64 = W(I, W_CG_AP);
   std::vector<double> b2(ncol), bn(ncol), rr(ncol), maxrr(ncol);
   std::vector<long> iters(ncol, 0);
   std::vector<double> pend(ncol, 0.0);  // alpha of a direction not yet added to x
   std::vector<int> active;
   const double target = stop_rsd * stop_rsd;
-  // |b - A x64|^2 / |b|^2 with r64 = b - A x64
+  // |b - A x64|^2 / |b|^2 with r = (b - A x64) / |b|
   auto true_residual = [&](int c) {
-    op_hermop<double>(*tp.colinv[c], ax64, x64[c], 1);
-    I.stats.hermop_fp64 += 1;
-    copy64(I, r64, b64[c]);
-    qdwf::launch_axpy<double2>(-1.0, ax64, r64, nd, I.stream);
-    check_launch();
-    return dev_norm2(I, r64) / b2[c];
+    return fp64_residual(I, *tp.colinv[c], b64[c], x64[c], tp.rat(tp.R, c), tp.rxh(), 1.0 / bn[c]) / b2[c];
   };
   for (int c = 0; c < ncol; ++c) {
     b2[c] = dev_norm2(I, b64[c]);
@@ -1516,7 +1507,6 @@ long cg_mixed_multi_s(Inv& I, int ncol, double2* const* b64, double2* const* x64
         if (rel > I.stats.true_residual) I.stats.true_residual = rel;
         continue;
       }
-      tp.set_r(r64, c, 1.0 / bn[c]);
     } else {
       tp.set_r(b64[c], c, 1.0 / bn[c]);  // x = 0: r = b
       rr[c] = maxrr[c] = 1.0;
@@ -1635,7 +1625,6 @@ long cg_mixed_multi_s(Inv& I, int ncol, double2* const* b64, double2* const* x64
             if (rel > I.stats.true_residual) I.stats.true_residual = rel;
             continue;  // column retired
           }
-          tp.set_r(r64, c, 1.0 / bn[c]);
           const int jf = hs.iters[i] - 1;  // the step of this replay that froze the column
           const int b = (k - jf) & 1;
           ru[b].push_back(c);
@@ -1697,7 +1686,6 @@ long cg_mixed_multi_s(Inv& I, int ncol, double2* const* b64, double2* const* x64
           if (rel > I.stats.true_residual) I.stats.true_residual = rel;
           continue;  // column retired
         }
-        tp.set_r(r64, c, 1.0 / bn[c]);
         rr_new[i] = rr_true;
         maxrr[c] = rr_true;
         step_alpha = 0.0;
@@ -1802,15 +1790,9 @@ bool use_three_phase(const Inv& I)
 
 double true_residual_fp64(Inv& I, const double2* x, const double2* b)
 {
-  double2* r = W(I, W_CG_R);
-  double2* ax = W(I, W_CG_AP);
-  op_hermop<double>(I, ax, x, 1);
-  I.stats.hermop_fp64 += 1;
-  copy64(I, r, b);
-  qdwf::launch_axpy<double2>(-1.0, ax, r, n64(I), I.stream);
-  check_launch();
+  const double r2 = fp64_residual(I, I, b, x);
   const double b2 = dev_norm2(I, b);
-  return b2 > 0 ? std::sqrt(dev_norm2(I, r) / b2) : 0.0;
+  return b2 > 0 ? std::sqrt(r2 / b2) : 0.0;
 }
 
 // The reference's is_checking_invert() (dslash.h:11-16, default true):
@@ -1824,18 +1806,36 @@ double residual_5d(Inv& I, const double2* x_e, const double2* x_o, const double2
 {
   double2* re = W(I, W_TMP);
   double2* ro = W(I, W_ITMP);
-  op_m_full(I, re, ro, x_e, x_o);
-  qdwf::launch_axpy<double2>(-1.0, dm_e, re, n64(I), I.stream);
-  qdwf::launch_axpy<double2>(-1.0, dm_o, ro, n64(I), I.stream);
-  check_launch();
-  const double num = dev_norm2(I, re) + dev_norm2(I, ro);
-  const double den = dev_norm2(I, dm_e) + dev_norm2(I, dm_o);
+  op_m_full(I, re, ro, x_e, x_o, dm_e, dm_o);
+  const double num = dev_norm2_sum(I, re, ro);
+  const double den = dev_norm2_sum(I, dm_e, dm_o);
   return den > 0 ? std::sqrt(num / den) : 0.0;
 }
 
 void note_residual_5d(Inv& I, double r)
 {
   if (r > I.stats.true_residual_5d) I.stats.true_residual_5d = r;
+}
+
+// set_odd_prec_field_sym2 (dslash.h:401-417): oep = M_ee^-1 dm_e and
+// b = Mpc^+ (dm_o - H P oep)
+void odd_prec_source(Inv& I, const double2* dm_e, const double2* dm_o, double2* oep, double2* b)
+{
+  double2* t = W(I, W_OP_T1);
+  m5<double>(I, oep, dm_e, MAT_MEE_INV);
+  m5<double>(I, t, oep, MAT_P);
+  hop<double>(I, b, t, 1, false, -1.0, dm_o, 0);
+  op_mpcdag<double>(I, b, b, 1);
+}
+
+// restore_field_from_odd_prec_sym2 (dslash.h:419-438): out_o = M_oo^-1 x_o
+// and out_e = oep - M_ee^-1 H P out_o
+void restore_column(Inv& I, const double2* x_o, const double2* oep, double2* out_e, double2* out_o)
+{
+  double2* tmp = W(I, W_TMP);
+  m5<double>(I, out_o, x_o, MAT_MEE_INV);
+  op_m_e_o<double>(I, tmp, out_o, 1);
+  m5<double>(I, out_e, tmp, MAT_MEE_INV, -1.0, oep, 1.0);
 }
 
 // invert_with_cg (dslash.h:440-530) on device halves; in_e/in_o: 5D source
@@ -1854,7 +1854,7 @@ long invert_halves(Inv& I, const double2* in_e, const double2* in_o, double2* ou
     copy64(I, dm_e, in_e);
     copy64(I, dm_o, in_o);
   }
-  const double dm_in_qnorm = dev_norm2(I, dm_e) + dev_norm2(I, dm_o);
+  const double dm_in_qnorm = dev_norm2_sum(I, dm_e, dm_o);
   if (dm_in_qnorm == 0.0) {
     zero64(I, out_e);
     zero64(I, out_o);
@@ -1863,13 +1863,7 @@ long invert_halves(Inv& I, const double2* in_e, const double2* in_o, double2* ou
   // set_odd_prec_field_sym2 (dslash.h:401-417)
   double2* out_e_p = W(I, W_OUT_EP);
   double2* in_o_p = W(I, W_IN_OP);
-  double2* tmp = W(I, W_TMP);
-  m5<double>(I, out_e_p, dm_e, MAT_MEE_INV);
-  op_m_e_o<double>(I, tmp, out_e_p, 2);
-  copy64(I, in_o_p, dm_o);
-  qdwf::launch_axpy<double2>(-1.0, tmp, in_o_p, n64(I), I.stream);
-  check_launch();
-  op_mpcdag<double>(I, in_o_p, in_o_p, 1);
+  odd_prec_source(I, dm_e, dm_o, out_e_p, in_o_p);
   double2* out_o_p = W(I, W_OUT_OP);
   zero64(I, out_o_p);
   long total_iter = 0;
@@ -1921,13 +1915,7 @@ long invert_halves(Inv& I, const double2* in_e, const double2* in_o, double2* ou
   }
   I.stats.total_iter += total_iter;
   if (true_rel > I.stats.true_residual) I.stats.true_residual = true_rel;
-  // restore_field_from_odd_prec_sym2 (dslash.h:419-438)
-  m5<double>(I, out_o, out_o_p, MAT_MEE_INV);
-  op_m_e_o<double>(I, tmp, out_o, 1);
-  m5<double>(I, W(I, W_ITMP), tmp, MAT_MEE_INV);
-  copy64(I, out_e, out_e_p);
-  qdwf::launch_axpy<double2>(-1.0, W(I, W_ITMP), out_e, n64(I), I.stream);
-  check_launch();
+  restore_column(I, out_o_p, out_e_p, out_e, out_o);
   if (g_checking_invert) note_residual_5d(I, residual_5d(I, out_e, out_o, dm_e, dm_o));
   return total_iter;
 }
@@ -2127,14 +2115,8 @@ double prepare_column(Inv& I, const double2* in_e, const double2* in_o, double2*
     copy64(I, dm_e, in_e);
     copy64(I, dm_o, in_o);
   }
-  const double q = dev_norm2(I, dm_e) + dev_norm2(I, dm_o);
-  double2* tmp = W(I, W_TMP);
-  m5<double>(I, oep, dm_e, MAT_MEE_INV);  // out_e' = M_ee^-1 (D_- in)_e
-  op_m_e_o<double>(I, tmp, oep, 2);
-  copy64(I, b, dm_o);
-  qdwf::launch_axpy<double2>(-1.0, tmp, b, n64(I), I.stream);
-  check_launch();
-  op_mpcdag<double>(I, b, b, 1);
+  const double q = dev_norm2_sum(I, dm_e, dm_o);
+  odd_prec_source(I, dm_e, dm_o, oep, b);
   return q;
 }
 
@@ -2146,18 +2128,6 @@ void out_e_p_of(Inv& I, const double2* in_e, const double2* in_o, double2* oep)
   if (I.dminus) op_d_minus(I, dm_e, W(I, W_DM_O), in_e, in_o);
   else copy64(I, dm_e, in_e);
   m5<double>(I, oep, dm_e, MAT_MEE_INV);
-}
-
-// restore_field_from_odd_prec_sym2 (dslash.h:419-438)
-void restore_column(Inv& I, const double2* x_o, const double2* oep, double2* out_e, double2* out_o)
-{
-  double2* tmp = W(I, W_TMP);
-  m5<double>(I, out_o, x_o, MAT_MEE_INV);
-  op_m_e_o<double>(I, tmp, out_o, 1);
-  m5<double>(I, W(I, W_ITMP), tmp, MAT_MEE_INV);
-  copy64(I, out_e, oep);
-  qdwf::launch_axpy<double2>(-1.0, W(I, W_ITMP), out_e, n64(I), I.stream);
-  check_launch();
 }
 
 // Multi-RHS driver of the mixed solvers: columns j < n, column j with the
@@ -2424,11 +2394,10 @@ long fermion_force_dev(Inv& I, const double2* phi, double stop_rsd, double2* for
 void build_matrices(Inv& I)
 {
   const int ls = I.ls;
-  std::vector<cd> bt(ls), ct(ls), negc(ls);
+  std::vector<cd> bt(ls), ct(ls);
   for (int s = 0; s < ls; ++s) {
     bt[s] = 1.0 + I.bs[s] * (4.0 - I.m5);  // dslash.cpp:617-621
     ct[s] = 1.0 - I.cs[s] * (4.0 - I.m5);
-    negc[s] = -I.cs[s];
   }
   std::vector<cd> ones(ls, 1.0), zeros(ls, 0.0);
   std::vector<cd> all((size_t)MAT_COUNT * 2 * ls * ls);
@@ -2440,10 +2409,8 @@ void build_matrices(Inv& I)
     const Mat mee_inv = mat_inv(mee, ls);
     const Mat pm = diag_plus(I.bs, I.cs, S, ls);
     const Mat k = mat_mul(pm, mee_inv, ls);
-    Mat negcm(ls * ls, 0.0);
-    for (int s = 0; s < ls; ++s) negcm[s * ls + s] = negc[s];
     const Mat list[MAT_COUNT] = {mee, mat_adj(mee, ls), mee_inv, mat_adj(mee_inv, ls), pm, mat_adj(pm, ls),
-                                 k, mat_adj(k, ls), negcm};
+                                 k, mat_adj(k, ls)};
     for (int m = 0; m < MAT_COUNT; ++m)
       std::memcpy(&all[((size_t)m * 2 + chi) * ls * ls], list[m].data(), sizeof(cd) * ls * ls);
   }
@@ -2465,13 +2432,15 @@ void build_matrices(Inv& I)
   I.mat32 = (cplx<float>*)dev_alloc(h32.size() * sizeof(cplx<float>));
   QDWF_HIP(hipMemcpy(I.mat64, h64.data(), h64.size() * sizeof(cplx<double>), hipMemcpyHostToDevice));
   QDWF_HIP(hipMemcpy(I.mat32, h32.data(), h32.size() * sizeof(cplx<float>), hipMemcpyHostToDevice));
-  std::vector<cplx<double>> b64(2 * ls);
+  std::vector<cplx<double>> b64(3 * ls);
   std::vector<cplx<float>> b32(2 * ls);
   for (int s = 0; s < ls; ++s) {
     b64[s].re = 1.0;
     b64[s].im = 0.0;
     b64[ls + s].re = ct[s].real();
     b64[ls + s].im = ct[s].imag();
+    b64[2 * ls + s].re = -I.cs[s].real();
+    b64[2 * ls + s].im = -I.cs[s].imag();
     b32[s].re = 1.0f;
     b32[s].im = 0.0f;
     b32[ls + s].re = (float)ct[s].real();

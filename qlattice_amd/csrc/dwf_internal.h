@@ -40,6 +40,7 @@ struct HopArgs {
   void* out;           // SoA spinor, parity eo_out
   const void* x;       // optional xpay operand (parity eo_out) or nullptr
   const cplx<T>* beta; // per-s xpay coefficients (device), used with x
+  const cplx<T>* gamma = nullptr;  // FP64: optional per-s factors of the hop term
   const void* links;   // 8-link layout (dwf_common.h)
   RhsSet cols;         // in/out/x are stacks of fields
   const void* cg;      // FP64: optional CgState64, nothing is done once it is done
@@ -213,6 +214,10 @@ inline int cg_residual_grid(int64_t n)
 {
   return (int)((n + 1023) / 1024 < kMaxCgResidualGrid ? (n + 1023) / 1024 : kMaxCgResidualGrid);
 }
+// r = scale (b - ax) in FP32 or FP16 storage (r may be null), block sums of
+// |b - ax|^2 into part; returns their number
+int launch_residual_d(const double2* b, const double2* ax, void* r, bool half, const LatGeo& g, int ls, double scale,
+                      double* part, hipStream_t st);
 void launch_cg_init_d(CgState64* st, double rr, double target, hipStream_t s);
 void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st);
 int64_t hop_m5d_blocks(const LatGeo& g, int ls);
