@@ -302,7 +302,8 @@ __device__ __forceinline__ void store_qs(typename SpinorIO<ST>::slot_t* __restri
 
 // HM: 0 FP32 arithmetic in the hop phase, 2 neighbour spinors of a thread in
 // flight; 1 FP16 arithmetic (hop_term_h2), 3 in flight; 5 waves per SIMD (fewer
-// where LDS has no room for them).
+// where LDS has no room for them), 6 in the plain FP16 hop, so that two blocks
+// of 64 sites fit a CU at Ls12 (33.5 against 35.2 us a column at 16^3x32).
 // FP32: bound by what it fetches, 0.41 ms for b = K H t at 24^3x64 Ls12.
 // Against batches of 4 spinors with 3 waves Mpc^+ Mpc takes 1924 instead of
 // 1947 us there, 176 instead of 184 at 16^3x32 Ls8, 543 instead of 579 at Ls24;
@@ -326,7 +327,8 @@ struct HopMode {
   static constexpr int km = SMAT ? 2 * LSMAX * LSMAX * (REAL && SB <= 16 ? 4 : 8) : 64 * SB;
   static constexpr int lds = (SMAT && hr > link ? hr : link) + km + 256;
   static constexpr int waves = (SB * LSMAX + 63) / 64 * (160 * 1024 / lds) / 4;
-  static constexpr int wpe = waves > 5 ? 5 : waves > 1 ? waves : 1;
+  static constexpr int cap = h2 && !SMAT ? 6 : 5;
+  static constexpr int wpe = waves > cap ? cap : waves > 1 ? waves : 1;
 };
 
 template <class ST, int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT, bool SMAT, int HM>
