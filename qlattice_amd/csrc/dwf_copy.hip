@@ -9,7 +9,6 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 #include "dwf_internal.h"
@@ -42,7 +41,7 @@ void run_threads(int n, Work&& work)
   int started = 1;  // (work(0) is this thread's)
   try {
     for (; started < n; ++started) th.emplace_back(work, started);
-  } catch (const std::system_error&) {
+  } catch (...) {  // (no more threads: the rest runs here)
   }
   work(0);
   for (int t = started; t < n; ++t) work(t);
