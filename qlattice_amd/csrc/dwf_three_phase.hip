@@ -309,7 +309,7 @@ __device__ __forceinline__ void store_qs(typename SpinorIO<ST>::slot_t* __restri
 // 1947 us there, 176 instead of 184 at 16^3x32 Ls8, 543 instead of 579 at Ls24;
 // batches with 4 waves spill.
 // The FP16 kernels are bound by VALU issue (70-76% busy in counters).  Site
-// places from the neighbour table, power-of-two scales, one v_max3 per pair,
+// places from the neighbour table, scales by v_rcp, one v_max3 per pair,
 // first terms assigned instead of added to zeros and streamed inputs taken
 // without an unscaled copy leave 1001 of 1216 instructions in b = K H t, 833
 // of 999 in the plain hop and 1336 of 1658 in the hop with the dot product:
