@@ -524,9 +524,12 @@ void hop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, 
          T alpha = 1, const typename Prec<T>::slot* x = nullptr, int beta = 0, const qdwf::RhsSet* cols = nullptr,
          const qdwf::CgState64* cg = nullptr, const cplx<T>* gamma = nullptr)
 {
-  qdwf::HopArgs<T> a;
-  a.cg = cg;
-  a.gamma = gamma;
+  constexpr bool kDouble = std::is_same<T, double>::value;  // (cg and gamma: FP64 only)
+  std::conditional_t<kDouble, qdwf::HopDArgs, qdwf::HopArgs<T>> a;
+  if constexpr (kDouble) {
+    a.cg = cg;
+    a.gamma = gamma;
+  }
   a.cols = cols ? *cols : one_col();
   a.geo = I.geo;
   a.ls = I.ls;
@@ -538,7 +541,7 @@ void hop(Inv& I, typename Prec<T>::slot* out, const typename Prec<T>::slot* in, 
   a.x = x;
   a.beta = Prec<T>::beta(I, beta);
   a.links = Prec<T>::links(I);
-  if constexpr (std::is_same<T, double>::value) qdwf::launch_hop_d(a, dag, I.stream);
+  if constexpr (kDouble) qdwf::launch_hop_d(a, dag, I.stream);
   else qdwf::launch_hop<T>(a, dag, I.hop_spt32, I.stream);
   check_launch();
 }

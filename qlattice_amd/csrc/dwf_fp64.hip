@@ -383,11 +383,11 @@ __device__ __forceinline__ void stage_links_d(double2 (*sl)[SB], int (*nbs)[SB],
 // behind the last direction's products: inside Mpc^+ Mpc 98 against 109 us at
 // 16^3x32 Ls8, 10.2 against 11.8 us at 8^3x16 Ls8.
 template <int SB, int NW, bool DAG, bool XPAY, bool NT>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB == 64 ? 2 : 3))) k_hop_d(HopArgs<double> a)
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB == 64 ? 2 : 3))) k_hop_d(HopDArgs a)
 {
   __shared__ double2 sl[72][SB];
   __shared__ int nbs[8][SB];
-  if (a.cg && ((const CgState64*)a.cg)->done) return;
+  if (a.cg && a.cg->done) return;
   const int64_t h0 = xcd_logical_block(blockIdx.x, (int64_t)gridDim.x) * SB;
   stage_links_d<SB, (72 * SB + 64 * NW - 1) / (64 * NW)>(sl, nbs, (const double2*)a.links, a.geo, h0, a.eo_out);
   __syncthreads();
@@ -440,7 +440,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB
 }
 
 template <int SB, int NW>
-static void launch_hop_d_sb(const HopArgs<double>& a, bool dag, hipStream_t st)
+static void launch_hop_d_sb(const HopDArgs& a, bool dag, hipStream_t st)
 {
   const dim3 grid((unsigned)((a.geo.vh + SB - 1) / SB));
   const dim3 blk(64 * NW);
@@ -454,7 +454,7 @@ static void launch_hop_d_sb(const HopArgs<double>& a, bool dag, hipStream_t st)
   if (dag && xpay && nt) hipLaunchKernelGGL((k_hop_d<SB, NW, true, true, true>), grid, blk, 0, st, a);
 }
 
-void launch_hop_d(const HopArgs<double>& a, bool dag, hipStream_t st)
+void launch_hop_d(const HopDArgs& a, bool dag, hipStream_t st)
 {
   // 64 sites: a gather shifted by one site then touches 9 cache lines per KB
   // instead of 12 (24^3x64 Ls12: 0.81 against 0.88 ms; 16^3x32 Ls8: 64
