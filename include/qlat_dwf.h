@@ -311,7 +311,8 @@ int qlat_dwf_multiply_m_dwf_qed(const int total_site[4], int ls, const double* g
                                 const double* wick, int is_dagger, double* out, const double* in);
 /* cg_with_m_dwf_qed (qed.cpp:178-261): M^+ M out = in (M M^+ when
  * is_dagger) from the initial guess in out; iter = iterations or
- * max_num_iter + 1. */
+ * max_num_iter + 1 (also when the residual stops being finite, as for a zero
+ * source; out is then no solution). */
 int qlat_dwf_cg_with_m_dwf_qed(const int total_site[4], int ls, const double* gf1, double mass, double m5,
                                const double* wick, int is_dagger, double stop_rsd, long max_num_iter, double* out,
                                const double* in, long* iter);

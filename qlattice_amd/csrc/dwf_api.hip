@@ -3103,7 +3103,8 @@ double qed_norm2(const double2* x, int64_t n, double* part, double* red)
 
 // cg_with_m_dwf_qed (qed.cpp:178-261): M_{!d} M_{d} x = b from the guess in
 // x, with the scalars on the device and the iterations queued ahead as in
-// cg_fp64
+// cg_fp64.  A residual that is no longer finite (a zero source has alpha =
+// 0/0) ends the iterations, since none after it can converge.
 long qed_cg(const QedCall& q, double2* x, const double2* b, bool dagger, double stop_rsd, long max_num_iter)
 {
   QDWF_REQUIRE(stop_rsd >= 0.0 && max_num_iter >= 0, "invalid stop_rsd or max_num_iter");
@@ -3146,7 +3147,7 @@ long qed_cg(const QedCall& q, double2* x, const double2* b, bool dagger, double 
     qdwf::launch_qed_iter(ia, nullptr);
     check_launch();
   });
-  return end.done ? (long)end.iter : max_num_iter + 1;
+  return end.done == 1 ? (long)end.iter : max_num_iter + 1;
 }
 
 }  // namespace

@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256) k_qed_direction(QedIterArgs a, int nrnorm
     return;
   }
   const double rr = sum_parts(a.rnorm, nrnorm);
-  const CgState64 next{rr, st.target, 0.0, st.iter + 1, rr <= st.target ? 1 : 0};
+  const CgState64 next{rr, st.target, 0.0, st.iter + 1, !isfinite(rr) ? 2 : rr <= st.target ? 1 : 0};
   if (first) {
     a.st[1 - a.slot] = next;
     *a.host = next;

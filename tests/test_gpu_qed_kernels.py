@@ -43,3 +43,21 @@ def test_cg_limits(limit):
     ref, it_ref = Q.cg_with_m_dwf_qed(x, g, 0.1, 1.0, ls, site, wick, False, 1e-10, limit)
     assert it == it_ref == limit + 1
     assert rel(sol, ref) < 1e-11
+
+
+@pytest.mark.parametrize("bad", [0.0, np.nan, 1e200])
+def test_cg_ends_where_the_residual_is_not_finite(bad):
+    """A zero source (alpha = 0/0), a NaN and a norm that overflows: no later
+    iteration can converge, so the solve returns at once, with the count that
+    says so, whatever its limit (at 1e9 iterations it would take hours)."""
+    site, ls, limit = (3, 4, 2, 5), 4, 10**9
+    g, wick, x = fields(site, ls, 9)
+    x[7, 1, 2] = bad
+    if bad == 0.0:
+        x[:] = 0.0
+    print(f"\n[gpu] QED CG, source with {bad}", flush=True)
+    sol, it = q.cg_with_m_dwf_qed(x, g, 0.1, 1.0, ls, site, wick, False, 1e-10, limit)
+    assert it == limit + 1
+    if bad == 0.0:
+        out, it = q.invert_dwf_qed(x[:, 0], g, 0.1, 1.0, ls, site, wick, False, 1e-10, limit)
+        assert it == limit + 1
