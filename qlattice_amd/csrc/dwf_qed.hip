@@ -1,6 +1,7 @@
 // The QED domain-wall operator on full (not even-odd) 5D fields [site][s][4]
 // (multiply_m_dwf_qed, qed.cpp:263-411) and the vector updates of its CG.
 #include "dwf_internal.h"
+#include "dwf_rules.h"
 
 namespace qdwf {
 
@@ -56,7 +57,9 @@ template <bool DAG, bool DOT>
 __global__ void __launch_bounds__(kBlasBlock) k_qed_m(QedArgs a)
 {
   if (a.cg && a.cg->done) return;
-  const int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x;
+  const int64_t blk = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (blk * kBlasBlock >= a.nelem) return;  // (of a grid spread over y)
+  const int64_t i = blk * kBlasBlock + threadIdx.x;
   double dot = 0.0;
   if (i < a.nelem) {
     const int ls = a.ls, r = (int)(i & 3);
@@ -147,7 +150,7 @@ __global__ void __launch_bounds__(kBlasBlock) k_qed_m(QedArgs a)
   }
   if (DOT) {
     dot = block_sum<kBlasBlock / 64>(dot);
-    if (threadIdx.x == 0) a.part[blockIdx.x] = dot;
+    if (threadIdx.x == 0) a.part[blk] = dot;
   }
 }
 
@@ -155,7 +158,8 @@ int64_t qed_m_blocks(const QedArgs& a) { return (a.nelem + kBlasBlock - 1) / kBl
 
 void launch_qed_m(const QedArgs& a, hipStream_t st)
 {
-  const dim3 grid((unsigned)qed_m_blocks(a)), blk(kBlasBlock);
+  const Grid2 g = split_blocks(qed_m_blocks(a), kBlasBlock);
+  const dim3 grid(g.x, g.y), blk(kBlasBlock);
   if (a.dagger) {
     if (a.dotp) hipLaunchKernelGGL((k_qed_m<true, true>), grid, blk, 0, st, a);
     else hipLaunchKernelGGL((k_qed_m<true, false>), grid, blk, 0, st, a);

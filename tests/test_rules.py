@@ -1,0 +1,48 @@
+"""The host code's rules on sizes (dwf_rules.h, plain C++), compiled here and
+called through ctypes."""
+
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include "dwf_rules.h"
+extern "C" void split_blocks(int64_t nblk, int block, uint32_t* xy)
+{
+  const qdwf::Grid2 g = qdwf::split_blocks(nblk, block);
+  xy[0] = g.x;
+  xy[1] = g.y;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(SOURCE)
+    lib = str(d / "librules.so")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-I", os.path.join(ROOT, "qlattice_amd", "csrc"),
+                    str(d / "rules.cpp"), "-o", lib], check=True)
+    return ctypes.CDLL(lib)
+
+
+@pytest.mark.parametrize("nelem", [1, 256, 257, 2**32 - 256, 2**32 - 255, 2**32, 2**32 + 4, 3 * 2**32, 2**35 + 12])
+def test_a_launch_stays_below_the_grid_limit(rules, nelem):
+    """128^3 x 64 Ls 8 has 2^32 QED elements: one thread each is one more than
+    a grid dimension takes."""
+    nblk = (nelem + 255) // 256
+    xy = (ctypes.c_uint32 * 2)()
+    rules.split_blocks(ctypes.c_int64(nblk), 256, xy)
+    x, y = xy
+    assert x * 256 < 2**32 and y < 65536
+    assert nblk <= x * y < nblk + y
+    if nelem <= 2**32 - 256:
+        assert y == 1
