@@ -30,6 +30,7 @@
 
 #include "../../include/qlat_dwf.h"
 #include "dwf_internal.h"
+#include "dwf_rules.h"
 
 using qdwf::cplx;
 using qdwf::LatGeo;
@@ -2539,25 +2540,20 @@ int qlat_dwf_inverter_create(qlat_dwf_inverter** out, const int total_site[4], c
     I->geo.xh = total_site[0] / 2;
     // device site order: tiles of `by` rows in y and `bz` planes in z, each
     // swept in t (dwf_common.h); by = Y, bz = Z is the reference order.
-    // Defaults: by = the divisor of Y closest to 6, bz = the divisor of Z
-    // closest to 8: a t step is then short enough for the L2 to keep the
-    // neighbouring time slices.  Mpc^+ Mpc at 24^3x64 Ls12, bz = 24 against
-    // 12 and 6: FP64 4.21, 3.90, 3.83 ms, FP32 2.01, 1.89, 1.92 ms, FP16
-    // storage (12 columns, per column) 1.24, 1.12, 1.13 ms; 16^3x32 Ls12,
-    // bz = 16 against 8: 585, 554 us (FP64).
+    // Defaults: by = the divisor of Y closest to 6, bz by z_tile.
     // QLAT_DWF_TILE_Y / QLAT_DWF_TILE_Z override the defaults.
-    auto tile_of = [](int n, int pref, const char* env) {
-      int b = n;
-      for (int d = 1; d <= n; ++d)
-        if (n % d == 0 && std::abs(d - pref) < std::abs(b - pref)) b = d;
+    int by = total_site[1];
+    for (int d = 1; d <= total_site[1]; ++d)
+      if (total_site[1] % d == 0 && std::abs(d - 6) < std::abs(by - 6)) by = d;
+    auto tile_of = [](int n, int b, const char* env) {
       if (const char* e = std::getenv(env)) {
         const int v = std::atoi(e);
         if (v > 0 && n % v == 0) b = v;
       }
       return b;
     };
-    I->geo.by = tile_of(total_site[1], 6, "QLAT_DWF_TILE_Y");
-    I->geo.bz = tile_of(total_site[2], 8, "QLAT_DWF_TILE_Z");
+    I->geo.by = tile_of(total_site[1], by, "QLAT_DWF_TILE_Y");
+    I->geo.bz = tile_of(total_site[2], qdwf::z_tile(I->geo.xh, I->geo.by, total_site[2]), "QLAT_DWF_TILE_Z");
     I->geo.vh = V / 2;
     I->geo.stride = (I->geo.vh + qdwf::kStrideAlign - 1) / qdwf::kStrideAlign * qdwf::kStrideAlign;
     I->geo.dxh = qdwf::make_fastdiv((unsigned)I->geo.xh);
