@@ -1148,22 +1148,7 @@ void deflate_dev(Inv& I, double2* out, const double2* in, int eo)
   check_launch();
 }
 
-// Sites per block of the three-phase kernels where the autotuner does not
-// choose them (single columns, fixed tiles): 16, the smallest block of whole
-// waves, and 32 where Ls is no multiple of 4.  Solves of one column, 16
-// against 32 sites: FP32 24^3x64 Ls12 0.83 against 0.93 s, 16^3x32 Ls12 95
-// against 108 ms and Ls16 128 against 144 ms, FP16 storage 16^3x32 Ls12 68
-// against 74 ms, 8^3x16 Ls12 11.4 against 12.2 ms.  From 16^3x32 up Ls 8
-// keeps 32 (56.7 against 58.0 ms: blocks of two waves otherwise) and Ls 24
-// takes 8 (216 against 223 ms: three blocks of LDS more per CU).
-int default_sb(const Inv& I)
-{
-  if (I.tp_sb) return I.tp_sb;
-  const bool large = I.geo.vh >= 1 << 16;
-  if (large && I.ls == 8) return 32;
-  if (large && I.ls == 24) return 8;
-  return I.ls % 4 ? 32 : 16;
-}
+int default_sb(const Inv& I) { return I.tp_sb ? I.tp_sb : qdwf::three_phase_sites(I.ls, I.geo.vh); }
 
 struct ThreePhase {
   Inv& I;

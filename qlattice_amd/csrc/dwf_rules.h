@@ -46,4 +46,27 @@ inline int z_tile(int xh, int by, int nz)
   return best;
 }
 
+// Sites per block of the three-phase kernels where the autotuner does not
+// choose them (single columns, fixed tiles), half volume vh.  16 makes whole
+// waves of four rows, with the s-matrix phase on the matrix cores; Ls that is
+// no multiple of 4 needs 32.  Mpc^+ Mpc of one column, us:
+//   Ls 12, 16 against 32 sites: FP32 42 / 46 at 8^3x16, 262 / 267 at 16^3x32,
+//     FP16 storage 37 / 41 and 166 / 179; 20^3x40 FP32 742 / 706
+//   Ls 16: FP32 48 / 55 and 326 / 326, FP16 storage 42 / 48 and 201 / 210
+//   Ls 8, where a block of 16 sites is only two waves: FP32 38.1 / 38.6 at
+//     8^3x16, 86 / 79 at 12^3x24, 188 / 174 at 16^3x32, FP16 storage 34.3 /
+//     34.6, 65 / 60 and 123 / 115, with four columns 51 / 50, 152 / 144, 388 /
+//     369; 16 is ahead only in FP32 at some 300 blocks of 32 (12^4: 55 / 58)
+//   Ls 24, 16 against 8 sites (six waves and 41 KB of LDS against three and
+//     23 KB, so three blocks a CU against six): FP32 57 / 63 at 8^3x16, 89 /
+//     96 at 8^3x32, 124 / 124 at 12^4, 172 / 153 at 12^3x16, 577 / 525 at
+//     16^3x32, FP16 storage 49 / 53, 69 / 72, 96 / 91, 136 / 109 and 422 /
+//     360: 8 from more than two blocks of 16 sites a CU on
+inline int three_phase_sites(int ls, int64_t vh)
+{
+  if (ls == 8) return 32;
+  if (ls == 24) return vh > 2 * 256 * 16 ? 8 : 16;
+  return ls % 4 ? 32 : 16;
+}
+
 }  // namespace qdwf

@@ -18,6 +18,7 @@ extern "C" void split_blocks(int64_t nblk, int block, uint32_t* xy)
   xy[0] = g.x;
   xy[1] = g.y;
 }
+extern "C" int three_phase_sites(int ls, int64_t vh) { return qdwf::three_phase_sites(ls, vh); }
 extern "C" int z_tile(int xh, int by, int nz) { return qdwf::z_tile(xh, by, nz); }
 """
 
@@ -63,3 +64,17 @@ def test_z_tiles_keep_whole_lines(rules, nz, by):
         assert max(b * b / 97, 97 / (b * b)) <= max(nz * nz / 97, 97 / (nz * nz))
     assert [rules.z_tile(8, 4, 16), rules.z_tile(12, 6, 24), rules.z_tile(16, 4, 32)] == [8, 12, 8]
     assert [rules.z_tile(10, 5, 20), rules.z_tile(14, 7, 28)] == [20, 4]
+
+
+@pytest.mark.parametrize("ls", [6, 8, 10, 12, 14, 16, 20, 24])
+def test_sites_per_block_have_a_kernel(rules, ls):
+    """Whole waves and the sites the kernels are built for at this Ls; 32 at Ls
+    8 on every lattice (blocks of 16 lost up to 10% below 16^3x32)."""
+    for vh in (8, 256, 4096, 8192, 8200, 13824, 65535, 65536, 442368):
+        sb = rules.three_phase_sites(ls, ctypes.c_int64(vh))
+        assert sb in ((8, 16) if ls == 24 else (16, 32) if ls <= 16 else (16,))
+        assert sb * ls % 64 == 0
+        if ls == 8:
+            assert sb == 32
+        if ls == 24:
+            assert sb == (8 if vh > 8192 else 16)
