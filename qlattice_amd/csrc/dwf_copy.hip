@@ -12,6 +12,7 @@
 #include <thread>
 #include <vector>
 #include "dwf_internal.h"
+#include "dwf_rules.h"
 
 namespace qdwf {
 namespace {
@@ -24,11 +25,12 @@ constexpr int kCopyThreads = 4;
 // below two pieces nothing overlaps: the runtime's copy
 constexpr size_t kRingMin = 2 * kPiece;
 
-// One ring per process, used by one transfer at a time and given back with
-// the last inverter.
+// One ring per process, made when ring_pays says so, used by one transfer at
+// a time and given back with the last inverter.
 struct Ring {
   std::mutex mu;
   char* buf = nullptr;
+  size_t moved = 0;  // bytes that went without it
   int users = 0;
 } g_ring;
 
@@ -49,7 +51,8 @@ void run_threads(int n, Work&& work)
 }
 
 // A transfer through the ring; false: it is for the runtime's copy (small,
-// not pageable, another thread's transfer in the ring, no pinned memory).
+// not pageable, too early to make the ring, another thread's transfer in it,
+// no pinned memory).
 bool ring_copy(int device, hipStream_t st, char* dev, char* host, size_t bytes, bool in, size_t ring_min,
                hipError_t* err)
 {
@@ -59,10 +62,14 @@ bool ring_copy(int device, hipStream_t st, char* dev, char* host, size_t bytes, 
   else if (at.type != hipMemoryTypeUnregistered) return false;
   std::unique_lock<std::mutex> lock(g_ring.mu, std::try_to_lock);
   if (!lock.owns_lock() || !g_ring.users) return false;
-  if (!g_ring.buf && hipHostMalloc((void**)&g_ring.buf, kCopyThreads * 2 * kPiece, hipHostMallocPortable) != hipSuccess) {
-    (void)hipGetLastError();
-    g_ring.buf = nullptr;
-    return false;
+  if (!g_ring.buf) {
+    g_ring.moved += bytes;
+    if (!ring_pays(bytes, g_ring.moved)) return false;
+    if (hipHostMalloc((void**)&g_ring.buf, kCopyThreads * 2 * kPiece, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      g_ring.buf = nullptr;
+      return false;
+    }
   }
   const size_t np = (bytes + kPiece - 1) / kPiece;
   const unsigned hc = std::thread::hardware_concurrency();
@@ -129,8 +136,9 @@ void copy_ring_retain()
 void copy_ring_release()
 {
   std::lock_guard<std::mutex> lock(g_ring.mu);
-  if (--g_ring.users > 0 || !g_ring.buf) return;
-  (void)hipHostFree(g_ring.buf);
+  if (--g_ring.users > 0) return;
+  g_ring.moved = 0;
+  if (g_ring.buf) (void)hipHostFree(g_ring.buf);
   g_ring.buf = nullptr;
 }
 
