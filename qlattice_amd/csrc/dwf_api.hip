@@ -789,14 +789,6 @@ cd dev_dot(Inv& I, const S* a, const S* b, int64_t n)
   sync(I);
   return cd(I.red_map[0], I.red_map[1]);
 }
-template <class S>
-double dev_cg_update(Inv& I, double alpha, const S* p, const S* ap, S* x, S* r, int64_t n)
-{
-  qdwf::launch_cg_update<S>(alpha, p, ap, x, r, n, I.part, I.red_map_dev, I.stream);
-  check_launch();
-  sync(I);
-  return I.red_map[0];
-}
 void copy64(Inv& I, double2* dst, const double2* src)
 {
   if (dst != src) QDWF_HIP(hipMemcpyAsync(dst, src, field64_bytes(I), hipMemcpyDeviceToDevice, I.stream));

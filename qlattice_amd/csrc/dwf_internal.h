@@ -393,7 +393,6 @@ void launch_axpy_site(double alpha, const void* p, void* x, int ls, int64_t n5, 
 // FP64 blocked field <-> FP16 column over n5 = stride * ls 5D sites
 void launch_d2h(const double2* in, uint4* out, int ls, int64_t n5, double scale, hipStream_t st);
 void launch_h2d(const uint4* in, double2* out, int ls, int64_t n5, int acc, double scale, hipStream_t st);
-void launch_hop_h16(const HopArgs<float>& a, bool dag, hipStream_t st);
 template <class T>
 void launch_m5(const M5Args<T>& a, hipStream_t st);
 // the FP64 s-matrix (one column: cols ignored; no dotp)
@@ -402,7 +401,6 @@ template <class T>
 void launch_cg_step(const CgStepArgs<T>& a, hipStream_t st);
 template <class S>
 void launch_axpy_norm(double a, const S* ap, S* r, int64_t n, double* part, double* out, hipStream_t st);
-void launch_reduce(const double* part, int nblk, int nv, double* out, hipStream_t st);
 // out[i] = sum_b part[i*nblk + b], i < nrows
 void launch_reduce_rows(const double* part, int nblk, int nrows, double* out, hipStream_t st);
 template <class S>
@@ -420,9 +418,6 @@ template <class S>
 void launch_axpy(double a, const S* x, S* y, int64_t n, hipStream_t st);
 template <class S>
 void launch_xpay(const S* x, double a, S* y, int64_t n, hipStream_t st);
-template <class S>
-void launch_cg_update(double a, const S* p, const S* ap, S* x, S* r, int64_t n, double* part, double* out,
-                      hipStream_t st);
 
 void launch_copy(const float4* x, float4* y, int64_t n, hipStream_t st);
 // FP64 <-> FP32 blocked fields: out = scale * in (d2f); out (+)= scale * in (f2d, acc = 1 adds)

@@ -221,8 +221,6 @@ void launch_hop(const HopArgs<T>& a, bool dag, int spt, hipStream_t st)
 
 template void launch_hop<float>(const HopArgs<float>&, bool, int, hipStream_t);
 
-void launch_hop_h16(const HopArgs<float>& a, bool dag, hipStream_t st) { launch_hop_lds<Half16, 4, false>(a, dag, st); }
-
 // ============================================================ hop + M5
 // Fused out = alpha * Mat (H in) + beta * x for FP32 fields, where Mat is a
 // dense Ls x Ls per-chirality s-matrix (the K = P M_ee^-1 of the Schur
@@ -1346,11 +1344,6 @@ __device__ __forceinline__ void slot_dot(const double2& a, const double2& b, dou
   re += a.x * b.x + a.y * b.y;
   im += a.x * b.y - a.y * b.x;
 }
-__device__ __forceinline__ void slot_dot(const float4& a, const float4& b, double& re, double& im)
-{
-  re += (double)a.x * b.x + (double)a.y * b.y + (double)a.z * b.z + (double)a.w * b.w;
-  im += (double)a.x * b.y - (double)a.y * b.x + (double)a.z * b.w - (double)a.w * b.z;
-}
 
 __device__ __forceinline__ double2 slot_axpy(double a, double2 x, double2 y)
 {
@@ -1365,11 +1358,6 @@ __device__ __forceinline__ float4 slot_axpy(double a, float4 x, float4 y)
 __device__ __forceinline__ double2 slot_xpay(double2 x, double a, double2 y)
 {
   return make_double2(a * y.x + x.x, a * y.y + x.y);
-}
-__device__ __forceinline__ float4 slot_xpay(float4 x, double a, float4 y)
-{
-  const float f = (float)a;
-  return make_float4(f * y.x + x.x, f * y.y + x.y, f * y.z + x.z, f * y.w + x.w);
 }
 
 template <class S>
@@ -1486,22 +1474,6 @@ __global__ void __launch_bounds__(kBlasBlock) k_xpay(const S* __restrict__ x, do
 {
   for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock)
     y[i] = slot_xpay(x[i], a, y[i]);
-}
-
-// x += a p ; r -= a ap ; partial |r|^2
-template <class S>
-__global__ void __launch_bounds__(kBlasBlock) k_cg_update(double a, const S* __restrict__ p, const S* __restrict__ ap,
-                                                          S* __restrict__ x, S* __restrict__ r, int64_t n,
-                                                          double* part)
-{
-  double v[1] = {0.0};
-  for (int64_t i = (int64_t)blockIdx.x * kBlasBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlasBlock) {
-    x[i] = slot_axpy(a, p[i], x[i]);
-    const S rn = slot_axpy(-a, ap[i], r[i]);
-    r[i] = rn;
-    v[0] += slot_norm2(rn);
-  }
-  block_reduce_store<1>(v, part);
 }
 
 // r -= a ap ; partial |r|^2
@@ -1670,15 +1642,6 @@ void launch_xpay(const S* x, double a, S* y, int64_t n, hipStream_t st)
 {
   hipLaunchKernelGGL(k_xpay<S>, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, x, a, y, n);
 }
-template <class S>
-void launch_cg_update(double a, const S* p, const S* ap, S* x, S* r, int64_t n, double* part, double* out,
-                      hipStream_t st)
-{
-  const int g = blas_grid(n);
-  hipLaunchKernelGGL(k_cg_update<S>, dim3(g), dim3(kBlasBlock), 0, st, a, p, ap, x, r, n, part);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, st, part, g, 1, out);
-}
-
 void launch_copy(const float4* x, float4* y, int64_t n, hipStream_t st)
 {
   hipLaunchKernelGGL(k_copy<float4>, dim3(blas_grid(n)), dim3(kBlasBlock), 0, st, x, y, n);
@@ -1703,28 +1666,15 @@ int launch_axpy_norm_multi(const AxpyNormArgs<S>& a, double* out, hipStream_t st
   hipLaunchKernelGGL(k_reduce_rows, dim3(a.cols.n), dim3(1024), 0, st, a.part, g, out);
   return g;
 }
-template int launch_axpy_norm_multi<double2>(const AxpyNormArgs<double2>&, double*, hipStream_t);
 template int launch_axpy_norm_multi<float4>(const AxpyNormArgs<float4>&, double*, hipStream_t);
 
-void launch_reduce(const double* part, int nblk, int nv, double* out, hipStream_t st)
-{
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, st, part, nblk, nv, out);
-}
-template void launch_axpy_norm<double2>(double, const double2*, double2*, int64_t, double*, double*, hipStream_t);
 template void launch_axpy_norm<float4>(double, const float4*, float4*, int64_t, double*, double*, hipStream_t);
 
 template void launch_norm2<double2>(const double2*, int64_t, double*, double*, hipStream_t);
-template void launch_norm2<float4>(const float4*, int64_t, double*, double*, hipStream_t);
 template void launch_dot<double2>(const double2*, const double2*, int64_t, double*, double*, hipStream_t);
-template void launch_dot<float4>(const float4*, const float4*, int64_t, double*, double*, hipStream_t);
 template void launch_axpy<double2>(double, const double2*, double2*, int64_t, hipStream_t);
 template void launch_axpy<float4>(double, const float4*, float4*, int64_t, hipStream_t);
 template void launch_xpay<double2>(const double2*, double, double2*, int64_t, hipStream_t);
-template void launch_xpay<float4>(const float4*, double, float4*, int64_t, hipStream_t);
-template void launch_cg_update<double2>(double, const double2*, const double2*, double2*, double2*, int64_t,
-                                        double*, double*, hipStream_t);
-template void launch_cg_update<float4>(double, const float4*, const float4*, float4*, float4*, int64_t, double*,
-                                       double*, hipStream_t);
 
 void launch_d2f(const double2* in, float4* out, int ls, int64_t st, hipStream_t s, double scale)
 {
