@@ -433,10 +433,11 @@ void launch_prop_col_to_5d(const double2* src, double2* soa, const LatGeo& g, in
                            hipStream_t st);
 void launch_5d_to_prop_col(const double2* soa, double2* dst, const LatGeo& g, int ls, int eo, int col,
                            hipStream_t st);
-// l16 (optional): FP16 copy of the links, h16x2 (re, im) per element
-// Copies between host and device memory on a stream, complete for the host
-// array on return (the device side of copy_to_device is in stream order).
-// The staging ring lives while a retain is held.
+// Copies between host and device memory on a stream.  copy_to_host is
+// complete on return.  copy_to_device is in stream order on the device; a
+// pageable host array has been read on return, a pinned one may still be
+// read until the stream is synchronised.  Copies of at least ring_min bytes
+// may take the staging ring, which lives while a retain is held.
 void copy_ring_retain();
 void copy_ring_release();
 hipError_t copy_to_device(int device, hipStream_t st, void* dev, const void* host, size_t bytes, size_t ring_min = 0);
@@ -444,6 +445,7 @@ hipError_t copy_to_host(int device, hipStream_t st, void* host, const void* dev,
 // Device half-site index of the neighbours of every site: nbt[(p * 8 + d) *
 // stride + h], p the parity slot of h (0 even, 1 odd), d as in neighbour_of.
 void launch_neighbours(unsigned* nbt, const LatGeo& g, hipStream_t st);
+// l16 (optional): FP16 copy of the links, h16x2 (re, im) per element
 void launch_pack_gauge(const double2* gauge, double2* l64, float2* l32, unsigned* l16, const LatGeo& g,
                        hipStream_t st);
 
