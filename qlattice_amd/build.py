@@ -20,7 +20,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libqlat_dwf_hip.so")
 SOURCES = ["dwf_kernels.hip", "dwf_three_phase.hip", "dwf_fp64.hip", "dwf_layout.hip", "dwf_qed.hip", "dwf_copy.hip",
            "dwf_api.hip"]
-HEADERS = ["dwf_common.h", "dwf_internal.h", "dwf_rules.h", os.path.join("..", "..", "include", "qlat_dwf.h")]
+HEADERS = ["dwf_common.h", "dwf_internal.h", "dwf_rules.h", "dwf_cg_control.h",
+           os.path.join("..", "..", "include", "qlat_dwf.h")]
 
 INCLUDE = os.path.join(HERE, "..", "include")
 PYX = os.path.join(HERE, "_cdwf.pyx")

@@ -33,6 +33,7 @@
 #include "dwf_rules.h"
 
 using qdwf::cplx;
+using qdwf::CgControl;
 using qdwf::LatGeo;
 typedef std::complex<double> cd;
 
@@ -52,23 +53,13 @@ thread_local std::string g_last_error;
 // allocating (a guard against any path that would reach hipMalloc)
 thread_local int g_noalloc_depth = 0;
 
-struct HipError : std::runtime_error {
-  using std::runtime_error::runtime_error;
-};
+using qdwf::HipError;
 struct ArgError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 struct MemError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
-
-#define QDWF_HIP(expr)                                                                      \
-  do {                                                                                      \
-    hipError_t e_ = (expr);                                                                 \
-    if (e_ != hipSuccess)                                                                   \
-      throw HipError(std::string(#expr) + " failed: " + hipGetErrorString(e_) + " (" + \
-                     __FILE__ + ":" + std::to_string(__LINE__) + ")");                     \
-  } while (0)
 
 #define QDWF_REQUIRE(cond, msg)         \
   do {                                  \
@@ -163,70 +154,8 @@ enum Work64 {
 };
 enum Work32 { V_R, V_P, V_AP, V_X, V_T, V_T1, V_T2, V_T3, V_Y, W_COUNT32 };
 
-// A device-driven CG: the iteration's scalars live in two state slots on the
-// device (CgState64; an iteration reads slot it & 1 and writes the other),
-// and iterations are queued kCgAhead at a time, one group ahead of the group
-// the host waits for; those behind the converged one find its state and do
-// nothing.  No iteration waits for the host: 8^3x16 Ls8, 155 FP64 iterations
-// of 65 us, the solve 18.0 -> 10.7 ms with two host round trips less each.
-constexpr int kCgAhead = 2;
 constexpr int kRedDoubles = 4 * qdwf::kMaxRhs;  // reduction results of an inverter, its CG states behind them
 constexpr int64_t kMaxPrologueSums = 4096;  // more block sums go through a reduction kernel
-struct CgControl {
-  qdwf::CgState64* dev = nullptr;      // [2], the caller's
-  qdwf::CgState64* map = nullptr;      // mapped host copy of the newest state
-  qdwf::CgState64* map_dev = nullptr;
-  bool own_map = false;
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  // map_host null: a mapped page of its own
-  CgControl(void* dev_states, void* map_host, void* map_device)
-      : dev((qdwf::CgState64*)dev_states), map((qdwf::CgState64*)map_host), map_dev((qdwf::CgState64*)map_device)
-  {
-    try {
-      if (!map) {
-        QDWF_HIP(hipHostMalloc((void**)&map, sizeof(qdwf::CgState64), hipHostMallocMapped | hipHostMallocCoherent));
-        own_map = true;
-        QDWF_HIP(hipHostGetDevicePointer((void**)&map_dev, map, 0));
-      }
-      for (auto& e : ev) QDWF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    } catch (...) {
-      release();
-      throw;
-    }
-  }
-  ~CgControl() { release(); }
-  CgControl(const CgControl&) = delete;
-  CgControl& operator=(const CgControl&) = delete;
-  void release()
-  {
-    for (auto& e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (own_map && map) (void)hipHostFree(map);
-  }
-  // queue(slot) launches one iteration; returns the last state
-  template <class Queue>
-  qdwf::CgState64 run(double rr, double target, long max_num_iter, hipStream_t st, Queue&& queue)
-  {
-    *map = qdwf::CgState64{};
-    qdwf::launch_cg_init_d(dev, rr, target, st);
-    QDWF_HIP(hipGetLastError());
-    long queued = 0;
-    auto group = [&](hipEvent_t e) {
-      for (int j = 0; j < kCgAhead && queued < max_num_iter; ++j, ++queued) queue((int)(queued & 1));
-      QDWF_HIP(hipEventRecord(e, st));
-    };
-    group(ev[0]);
-    for (long g = 1;; ++g) {
-      const bool last = queued >= max_num_iter;
-      if (!last) group(ev[g & 1]);
-      QDWF_HIP(hipEventSynchronize(ev[(g - 1) & 1]));
-      if (last || *(volatile int*)&map->done) break;
-    }
-    QDWF_HIP(hipStreamSynchronize(st));  // the group queued behind
-    return *map;
-  }
-};
-
 // Tile width (columns per multi-RHS block) and sites per block of the
 // three-phase solver.
 struct TileChoice {

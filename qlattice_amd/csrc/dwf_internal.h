@@ -1,6 +1,7 @@
 // Internal interface between the kernel file and the C-ABI host code.
 #pragma once
 
+#include "dwf_cg_control.h"
 #include "dwf_common.h"
 
 namespace qdwf {
@@ -43,8 +44,6 @@ struct HopArgs {
   const void* links;   // 8-link layout (dwf_common.h)
   RhsSet cols;         // in/out/x are stacks of fields
 };
-
-struct CgState64;
 
 // The FP64 hop (launch_hop_d; one column: cols ignored).  What it takes more
 // is a type of its own: as members of HopArgs its two pointers cost the FP32
@@ -168,16 +167,6 @@ struct HopM5Args {
   FastDiv dncol;
 };
 
-// Scalars of the FP64 CG on the device, one slot for the even and one for
-// the odd iterations: an iteration reads slot it & 1 and writes the other.
-struct CgState64 {
-  double rr;      // |r|^2 before the iteration
-  double target;  // stop when |r|^2 <= target
-  double alpha;   // of the iteration (k_cg_residual_d)
-  int64_t iter;   // iterations done before this one
-  int done;       // 0 running, 1 converged, 2 non-finite
-};
-
 // FP64 fused hop + s-matrix (k_hop_m5d): out = alpha * Mat (H in) + beta * x
 // on one FP64 field; with dotp (dagger xpay form) part[block] = Re <dotp,
 // out>, hop_m5d_blocks of them.
@@ -226,7 +215,6 @@ inline int cg_residual_grid(int64_t n)
 // |b - ax|^2 into part; returns their number
 int launch_residual_d(const double2* b, const double2* ax, void* r, bool half, const LatGeo& g, int ls, double scale,
                       double* part, hipStream_t st);
-void launch_cg_init_d(CgState64* st, double rr, double target, hipStream_t s);
 void launch_cg_iter_d(const CgIterDArgs& a, hipStream_t st);
 int64_t hop_m5d_blocks(const LatGeo& g, int ls);
 
