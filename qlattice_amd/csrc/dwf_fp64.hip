@@ -60,8 +60,8 @@ struct SMat {
 
 // out = alpha Mat in (+ beta x): wave = 16 sites x kSmatComps components of
 // one chirality, block = 64 sites, blockIdx.y = the component group.
-// HBM bound, at the speed of a copy: 0.43 ms at 24^3x64 Ls12 (4.7 TB/s),
-// 31 us at 16^3x32 Ls8 and 4.3 us at 8^3x16 Ls12.  With one thread per site
+// HBM bound, at the speed of a copy: 0.36 to 0.42 ms at 24^3x64 Ls12 (4.9 to
+// 5.7 TB/s), 30 us at 16^3x32 Ls8 and 4.3 us at 8^3x16 Ls12.  With one thread per site
 // and slot looping over s on the vector units it was 0.61 ms, 46 us and
 // 14.3 us (57 us at 8^3x16 Ls24: a chain of scalar loads of the matrix).
 template <int LSMAX>
@@ -377,11 +377,12 @@ __device__ __forceinline__ void stage_links_d(double2 (*sl)[SB], int (*nbs)[SB],
 // out = alpha H in (+ beta_s x): block = SB sites, its waves take the rows
 // in turn.  Bound by the traffic beyond the 4 MB L2 of an XCD: the rows of
 // the sites in flight on its 32 CUs are larger than that, so a spinor is
-// fetched about three times per launch (24^3x64 Ls12, 0.81 ms).  Before the
-// links' loads were batched and the next spinor requested early: 0.88 ms, at
-// 16^3x32 Ls8 91 us (now 64), at 8^3x16 Ls12 28 us (now 7).  x is requested
-// behind the last direction's products: inside Mpc^+ Mpc 98 against 109 us at
-// 16^3x32 Ls8, 10.2 against 11.8 us at 8^3x16 Ls8.
+// fetched 4.3 times per launch at 24^3x64 Ls12 (0.78 ms, 7.6 TB/s in all), 2.5
+// times at 16^3x32 Ls8.  Before the links' loads were batched and the next
+// spinor requested early: 0.88 ms, at 16^3x32 Ls8 90 us (now 64), at 8^3x16
+// Ls12 28 us (now 7.7).  x is requested behind the last direction's products:
+// inside Mpc^+ Mpc 98 against 109 us at 16^3x32 Ls8, 10.2 against 11.8 us at
+// 8^3x16 Ls8.
 template <int SB, int NW, bool DAG, bool XPAY, bool NT>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(SB == 64 ? 2 : 3))) k_hop_d(HopDArgs a)
 {
@@ -457,7 +458,7 @@ static void launch_hop_d_sb(const HopDArgs& a, bool dag, hipStream_t st)
 void launch_hop_d(const HopDArgs& a, bool dag, hipStream_t st)
 {
   // 64 sites: a gather shifted by one site then touches 9 cache lines per KB
-  // instead of 12 (24^3x64 Ls12: 0.81 against 0.88 ms; 16^3x32 Ls8: 64
+  // instead of 12 (24^3x64 Ls12 without z tiles: 0.81 against 0.88 ms; 16^3x32 Ls8: 64
   // against 75 us), but it takes some 200 blocks to fill the chip (10x12^2x20
   // Ls12, 225 blocks: 25.4 against 28.5 us; 8^3x16 Ls12, 64 blocks: 14.1
   // against 7.0 us)
@@ -466,14 +467,15 @@ void launch_hop_d(const HopDArgs& a, bool dag, hipStream_t st)
 }
 
 // out = alpha Mat (H in) (+ beta x), with DOT also the block's part of
-// Re <dotp, out>.  Block = SB sites x
-// ls rows (rows up to a multiple of 4): thread (site, row) forms the hop of
-// its 5D site, the results go through LDS (over the links) one chirality
-// after the other (half the LDS), and the waves take the (component, 16
-// sites) pairs of the s-matrix product in turn.  Bound like k_hop_d: 0.93 ms
-// at 24^3x64 Ls12; 80 us at 16^3x32 Ls8 (97 with the product row by row from
-// LDS on the vector units), 11 us at 8^3x16 Ls8.  With x and the dot product
-// 117 and 14 us, 108 and 12 us with dotp requested before the s-matrix product.
+// Re <dotp, out>.  Block = SB sites x ls rows (rows up to a multiple of 4):
+// thread (site, row) forms the hop of its 5D site, the results go through LDS
+// (over the links) one chirality after the other (half the LDS), and the
+// waves take the (component, 16 sites) pairs of the s-matrix product in turn.
+// Bound like k_hop_d: 0.82 to 0.85 ms at 24^3x64 Ls12 (a spinor fetched 3.7
+// times, 6.3 TB/s beyond the L2); 80 us at 16^3x32 Ls8 (97 with the product row
+// by row from LDS on the vector units), 11 us at 8^3x16 Ls8.  With x and the
+// dot product 117 and 14 us, 108 and 12 us with dotp requested before the
+// s-matrix product.
 template <int SB, int LSMAX, bool DAG, bool XPAY, bool REAL, bool DOT, bool NT>
 __global__ void __launch_bounds__(SB * LSMAX) __attribute__((amdgpu_waves_per_eu(3))) k_hop_m5d(HopM5dArgs a)
 {

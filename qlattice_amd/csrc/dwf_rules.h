@@ -36,7 +36,8 @@ inline Grid2 split_blocks(int64_t nblk, int block)
 //   14^3x28, 7 planes 0.97 / 1.00 / 0.98
 // (the square of the middle is 97: 12 planes before 8, 7 before 14, none
 // before 4 at Z = 20).  On lattices that fit the L2s anyway (6x10x14x22) tiles
-// cost 1 to 2%, and the FP32 hop by itself 1 to 5%.
+// cost 1 to 2%, there and below the FP32 hop by itself 3 to 9%; the FP64 hop by
+// itself is faster with 8 planes at 24^3x64 Ls12 (0.73 against 0.78 ms).
 inline int z_tile(int xh, int by, int nz)
 {
   auto whole_lines = [&](int b) { return (int64_t)xh * by * b % 8 == 0; };

@@ -304,19 +304,23 @@ __device__ __forceinline__ void store_qs(typename SpinorIO<ST>::slot_t* __restri
 // flight; 1 FP16 arithmetic (hop_term_h2), 3 in flight; 5 waves per SIMD (fewer
 // where LDS has no room for them), 6 in the plain FP16 hop, so that two blocks
 // of 64 sites fit a CU at Ls12 (33.5 against 35.2 us a column at 16^3x32).
-// FP32: bound by what it fetches, 0.41 ms for b = K H t at 24^3x64 Ls12.
-// Against batches of 4 spinors with 3 waves Mpc^+ Mpc takes 1924 instead of
-// 1947 us there, 176 instead of 184 at 16^3x32 Ls8, 543 instead of 579 at Ls24;
-// batches with 4 waves spill.
-// The FP16 kernels are bound by VALU issue (70-76% busy in counters).  Site
+// FP32: bound by what it fetches, 0.39 ms for b = K H t at 24^3x64 Ls12.
+// Against batches of 4 spinors with 3 waves and links and hop results apart,
+// Mpc^+ Mpc of one column takes 0.98 of the time at 16^3x32 Ls8, 0.82 at Ls12
+// and 0.78 at 24^3x64 Ls12 (32-site blocks); at Ls8 b = K H t is 7 to 9% slower
+// from 20^3 up (four columns: Mpc^+ Mpc 1.02 to 1.03), whole solves are even.
+// Batches with 4 waves spill.
+// FP16: VALU 50-66% busy, 5.5 to 6.7 TB/s beyond the L2 and 76 to 99 requests
+// in flight per CU (24^3x64 Ls12, 4 columns): no one of them alone.  Site
 // places from the neighbour table, scales by v_rcp, one v_max3 per pair,
 // first terms assigned instead of added to zeros and streamed inputs taken
-// without an unscaled copy leave 1001 of 1216 instructions in b = K H t, 833
-// of 999 in the plain hop and 1336 of 1658 in the hop with the dot product:
-// the operator 188 -> 155 us a column at 16^3x32 Ls12 with 4 columns, 24^3x64
-// Ls12 with 12 columns 1237 -> 1105 us; rings of 3 instead of batches of 4
-// spinors leave 152 and 1086 us.  A budget of 6 waves spills in the s-matrix
-// phase: 1115 against 1093 us.
+// without an unscaled copy leave 961 of 1131 instructions a wave in b = K H t,
+// 782 of 969 in the plain hop and 1291 of 1519 in the hop with the dot
+// product.  With rings of 3 instead of batches of 4 spinors and the z tiles
+// the operator takes, per column, 0.92 of the time at 16^3x32 Ls12 (4 columns,
+// 158 -> 145 us), and at 24^3x64 Ls12 0.96 with 4 columns (1097 -> 1054 us), the
+// width that the autotuner takes there, 0.91 with 12 (1169 -> 1065 us).
+// A budget of 6 waves spills in the s-matrix phase.
 template <int HM, int SB, int LSMAX, bool REAL, bool SMAT>
 struct HopMode {
   static constexpr bool h2 = HM != 0;
