@@ -30,7 +30,7 @@ constexpr size_t kRingMin = 2 * kPiece;
 struct Ring {
   std::mutex mu;
   char* buf = nullptr;
-  size_t moved = 0;  // bytes that went without it
+  int without = 0;  // transfers that went without it
   int users = 0;
 } g_ring;
 
@@ -63,8 +63,10 @@ bool ring_copy(int device, hipStream_t st, char* dev, char* host, size_t bytes, 
   std::unique_lock<std::mutex> lock(g_ring.mu, std::try_to_lock);
   if (!lock.owns_lock() || !g_ring.users) return false;
   if (!g_ring.buf) {
-    g_ring.moved += bytes;
-    if (!ring_pays(bytes, g_ring.moved)) return false;
+    if (!ring_pays(bytes, g_ring.without)) {
+      ++g_ring.without;
+      return false;
+    }
     if (hipHostMalloc((void**)&g_ring.buf, kCopyThreads * 2 * kPiece, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
       g_ring.buf = nullptr;
@@ -137,7 +139,7 @@ void copy_ring_release()
 {
   std::lock_guard<std::mutex> lock(g_ring.mu);
   if (--g_ring.users > 0) return;
-  g_ring.moved = 0;
+  g_ring.without = 0;
   if (g_ring.buf) (void)hipHostFree(g_ring.buf);
   g_ring.buf = nullptr;
 }

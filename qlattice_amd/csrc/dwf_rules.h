@@ -72,16 +72,14 @@ inline int three_phase_sites(int ls, int64_t vh)
 }
 
 // Whether the staging ring of the host copies is to be made for a transfer of
-// `bytes` when the transfers without one have come to `moved` (this one
-// included).  Its 16 MB of pinned memory cost some 2 ms, which a single large
-// transfer or a few small ones win back: M_ee on host half fields on a new
-// inverter, first call with a ring against the runtime's copies 2.9 against
-// 1.2 ms at 12.6 MB, 3.6 against 2.4 ms at 25 MB, 5.4 against 3.1 ms at 32 MB,
-// 3.1 to 5.5 against 4.7 to 6.6 ms at 48 MB; the calls after it 0.90 / 1.11,
-// 1.50 / 2.2, 2.1 / 2.9 and 2.7 to 5.8 / 4.6 to 6.5 ms.
-inline bool ring_pays(size_t bytes, size_t moved)
-{
-  return bytes >= (size_t)40 << 20 || moved >= (size_t)128 << 20;
-}
+// `bytes` after `without` transfers that went without one.  Its 16 MB of
+// pinned memory cost up to 2 ms, more than one call on a small array wins
+// back: M_ee on host half fields on a new inverter, first call with a ring
+// against the runtime's copies 2.9 against 1.2 ms at 12.6 MB, 3.6 against 2.4
+// ms at 25 MB, 5.4 against 3.1 ms at 32 MB, 3.1 to 5.5 against 4.7 to 6.6 ms at
+// 48 MB; the calls after it 0.90 / 1.11, 1.50 / 2.2, 2.1 / 2.9 and 2.7 to 5.8 /
+// 4.6 to 6.5 ms.  So a first call, one array in and one out, goes without, and
+// the next one is taken for the second of many.
+inline bool ring_pays(size_t bytes, int without) { return bytes >= (size_t)40 << 20 || without >= 2; }
 
 }  // namespace qdwf

@@ -19,7 +19,7 @@ extern "C" void split_blocks(int64_t nblk, int block, uint32_t* xy)
   xy[1] = g.y;
 }
 extern "C" int three_phase_sites(int ls, int64_t vh) { return qdwf::three_phase_sites(ls, vh); }
-extern "C" int ring_pays(size_t bytes, size_t moved) { return qdwf::ring_pays(bytes, moved); }
+extern "C" int ring_pays(size_t bytes, int without) { return qdwf::ring_pays(bytes, without); }
 extern "C" int z_tile(int xh, int by, int nz) { return qdwf::z_tile(xh, by, nz); }
 """
 
@@ -81,16 +81,15 @@ def test_sites_per_block_have_a_kernel(rules, ls):
             assert sb == (8 if vh > 8192 else 16)
 
 
-def test_the_ring_waits_for_bytes(rules):
-    """A new inverter's first calls on small host arrays make no ring (its
-    pinned memory takes longer than their copies); a large array, or some calls
-    more, does."""
+def test_the_ring_waits_for_a_second_call(rules):
+    """A new inverter's first call on a small host array, one transfer in and
+    one out, makes no ring (its pinned memory takes longer than their copies);
+    the next one does, and a large array at once."""
     mb = 1 << 20
 
-    def pays(bytes_, moved):
-        return bool(rules.ring_pays(ctypes.c_size_t(bytes_), ctypes.c_size_t(moved)))
+    def pays(bytes_, without):
+        return bool(rules.ring_pays(ctypes.c_size_t(bytes_), without))
 
     for size in (4, 12, 18, 25, 32):
-        assert not pays(size * mb, 2 * size * mb)
-        assert pays(size * mb, 128 * mb)
-    assert pays(45 * mb, 45 * mb) and pays(96 * mb, 96 * mb)
+        assert not pays(size * mb, 0) and not pays(size * mb, 1) and pays(size * mb, 2)
+    assert pays(45 * mb, 0) and pays(96 * mb, 0)
